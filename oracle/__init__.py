@@ -53,7 +53,7 @@ def build(ref=None):
     """Compile the restatement (and oracle/_ref when the reference is present)."""
     subprocess.run(["make", "-s", "-C", HERE], check=True)
     if ref is None:
-        ref = os.path.isdir(REFERENCE)
+        ref = os.path.isdir(os.path.join(REFERENCE, "src"))
     if ref:
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
