@@ -4316,11 +4316,17 @@ struct DownLds {
 };
 
 // v as two f16 values hi = f16(v), lo = f16(v - hi) (v - hi is exact in fp32).
+// v is opaque to the compiler: a v that is a product would otherwise be
+// rounded to f16 straight from the exact product (v_fma_mixlo_f16) in one use
+// of hi and by way of fp32 in the other, and where the two roundings differ
+// hi + lo is off by 2^-11 of v (one super-block of y by up to 8e-5, measured).
 __device__ __forceinline__ void split_f16(const float (&v)[8], f16x8& hi, f16x8& lo) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    hi[j] = (_Float16)v[j];
-    lo[j] = (_Float16)(v[j] - (float)hi[j]);
+    float x = v[j];
+    asm("" : "+v"(x));
+    hi[j] = (_Float16)x;
+    lo[j] = (_Float16)(x - (float)hi[j]);
   }
 }
 

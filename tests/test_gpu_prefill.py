@@ -219,3 +219,22 @@ def test_prefill_large_down_scales(eng):
     finally:
         view[:] = good
         assert eng.refresh(1, units[1], 0, e0) == fa.OK
+
+
+def test_prefill_down_operand_parts_agree(eng):
+    """The down's two f16 parts of d*h sum to it: every token within 2e-6 of the
+    oracle. fp32 sums of 20 terms whose magnitudes add up to a few times the
+    result leave about 1e-6 at most; a hi part that one use rounds differently
+    from the other (2^-11 of one product) shows as 3e-6 and more in some token
+    of each of these chunks."""
+    hidden = 4096
+    lay = oracle.layout(hidden, fa.FMT_Q4KT)
+    for seed, blocks in ((5, (0, 1)), (6, (0, 1)), (7, (3,))):
+        load(eng, hidden, blocks)
+        rng = np.random.default_rng(seed)
+        experts, gates, x = chunk(rng, 40, hidden, rng.choice(512, 40, replace=False))
+        y = run_ok(eng, 0, experts, gates, x)
+        ref = oracle_rows(lay, blocks, 0, experts, gates, x)
+        for t in range(len(x)):
+            rc, err = oracle.compare(ref[t], y[t])
+            assert rc == 0 and err[0] <= 2e-6, (seed, t, err)
