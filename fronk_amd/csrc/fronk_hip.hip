@@ -3992,9 +3992,9 @@ __global__ void synth_kernel(uint8_t* __restrict__ dst, SliceShape routed, Slice
 // that each expert's weights are read once for all of its tokens and the
 // work is a contraction:
 //   prefill_split    (token): x as two f16 parts of x * 2^-e, once;
-//   prefill_gate_up  (tile, slice): a, u of up to 16 tokens over one slice's
-//                    32 neurons on f16 matrix cores (operands exact), then
-//                    gate*SiLU(a)*u;
+//   prefill_gate_up  (tile, slices): a, u of up to 64 tokens over the 32
+//                    neurons of up to four slices on f16 matrix cores
+//                    (operands exact), then gate*SiLU(a)*u;
 //   prefill_down     (tile, 512 outputs): the expert's down matrix over all
 //                    owned slices applied to the tile's h on f16 matrix
 //                    cores (A = sc*q exact, B = d*h in two exact parts), one
@@ -4013,7 +4013,9 @@ constexpr int kBatchThreads = 512;
 constexpr int kMaxBatchTokens = 4096;
 constexpr int kDownCols = 1024;          // outputs of one prefill_down workgroup
 
-struct BatchTile {                       // one routed expert and up to 16 of its tokens
+constexpr int kGateUpTiles = 4;          // 16-token tiles of one prefill_gate_up workgroup at most
+
+struct BatchTile {                       // one routed expert and up to 16 (gate/up: 64) of its tokens
   uint32_t expert, ntok, slot0, pad;
 };
 struct BatchSlot {                       // one (token, expert) of the chunk
@@ -4025,26 +4027,38 @@ struct BatchHeader {
   uint32_t nblk, layer, tiles_off, slots_off;
   uint32_t tokslot_off, x_off, total, experts;
   uint32_t nshared, shtiles, gu, dn;         // tokens with the shared expert, its tiles; routed formats
+  uint32_t gtiles_off, ngtiles;              // prefill_gate_up's tiles of the routed experts
+  uint32_t gslices, pad;                     // its slices per workgroup; 0: prefill_gate_up_few
   uint64_t slice_bytes, proj, shared_proj;
   uint64_t base[kBlocks];                // owned slices in ascending block order: the layer's base
 };
-static_assert(sizeof(BatchHeader) == 248, "batch header layout");
+static_assert(sizeof(BatchHeader) == 264, "batch header layout");
 constexpr uint32_t kNoSlot = ~0u;        // tokslot entry of a token without the shared expert
 struct BatchScratch {
   float* h;                              // [nslots][nblk * 32] gate * h
   float* part;                           // [nslots][hidden] per-(token, expert) partials
   float* y;                              // [tokens][hidden]
-  uint16_t* xh;                          // [tokens][super-block][2 parts][256] x' = x * 2^-e as f16 hi, lo
+  uint16_t* xh;                          // [tokens][super-block][512] x' = x * 2^-e as f16 hi, lo (xh_unit)
   float* dscale;                         // [tokens] 2^e
   float* dsum;                           // [tokens][super-block][8] sub-block sums of x'
+  uint16_t* xs;                          // [tokens][super-block][32] the same sums / 32 in three f16 parts
   uint32_t* status;
 };
 
 // x of the chunk for the f16 matrix cores: per token, x' = x * 2^-e with 2^e
 // chosen so that |x'| < 2^15, written as two f16 parts hi = f16(x'),
 // lo = f16(x' - hi) (22 significant bits; the f16 subnormal floor 2^-24 is
-// 2^-39 of the token's largest value), plus 2^e and the fp32 sum of each
-// 32-value sub-block of x' (for the min terms).
+// 2^-39 of the token's largest value), plus 2^e and the sum of each 32-value
+// sub-block of x' (for the min terms), in fp32 and, over 32, in three f16
+// parts (33 significant bits).
+// A token's super-block lies in 16-byte units of 8 values, in the order in
+// which prefill_gate_up's products read them: [half p][part][v][kg] holds
+// values 8v..8v+7 of sub-block 4p + kg, as 0, 2, 4, 6, 1, 3, 5, 7 (the order in
+// which a Q4_K dword's nibbles come out two at a time, nib_pair_at). The sums'
+// 16-byte unit kg is sub-block kg's parts hi, mid, lo, 0, then those of 4 + kg.
+__device__ __forceinline__ unsigned xh_unit(unsigned p, unsigned part, unsigned v, unsigned kg) {
+  return ((2 * p + part) * 4 + v) * 4 + kg;
+}
 __global__ __launch_bounds__(1024) void prefill_split(const uint8_t* __restrict__ plan, BatchScratch S) {
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
   const unsigned t = blockIdx.x, hidden = H.hidden, nsb = hidden / 256, v0 = 4 * threadIdx.x;
@@ -4071,32 +4085,86 @@ __global__ __launch_bounds__(1024) void prefill_split(const uint8_t* __restrict_
   const int e = max(E - 15, -126);
   const float v[4] = {x.x, x.y, x.z, x.w};
   float xs[4];
-  _Float16 hi[4], lo[4];
+  uint16_t hi[4], lo[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
     xs[j] = ok ? ldexpf(v[j], -e) : 0.f;
-    hi[j] = (_Float16)xs[j];
-    lo[j] = (_Float16)(xs[j] - (float)hi[j]);
+    const _Float16 h = (_Float16)xs[j];
+    hi[j] = __builtin_bit_cast(uint16_t, h);
+    lo[j] = __builtin_bit_cast(uint16_t, (_Float16)(xs[j] - (float)h));
   }
   float s = (xs[0] + xs[1]) + (xs[2] + xs[3]);
   s += __shfl_xor(s, 1, 64);
   s += __shfl_xor(s, 2, 64);
   s += __shfl_xor(s, 4, 64);   // the 8 threads of a 32-value sub-block
+  // Two threads hold a unit's 8 values: the even one writes its hi part, the
+  // odd one its lo part, each after one exchange of two dwords.
+  const bool odd = threadIdx.x & 1;
+  const uint32_t h0 = hi[0] | (uint32_t)hi[2] << 16, h1 = hi[1] | (uint32_t)hi[3] << 16;
+  const uint32_t l0 = lo[0] | (uint32_t)lo[2] << 16, l1 = lo[1] | (uint32_t)lo[3] << 16;
+  const uint32_t r0 = (uint32_t)__shfl_xor((int)(odd ? h0 : l0), 1, 64), r1 = (uint32_t)__shfl_xor((int)(odd ? h1 : l1), 1, 64);
   if (live) {
-    const unsigned sb = v0 / 256, pos = v0 % 256;
-    uint16_t* dst = S.xh + ((size_t)t * nsb + sb) * 512 + pos;
-    *reinterpret_cast<uint2*>(dst) = make_uint2(
-        (uint32_t)__builtin_bit_cast(uint16_t, hi[0]) | (uint32_t)__builtin_bit_cast(uint16_t, hi[1]) << 16,
-        (uint32_t)__builtin_bit_cast(uint16_t, hi[2]) | (uint32_t)__builtin_bit_cast(uint16_t, hi[3]) << 16);
-    *reinterpret_cast<uint2*>(dst + 256) = make_uint2(
-        (uint32_t)__builtin_bit_cast(uint16_t, lo[0]) | (uint32_t)__builtin_bit_cast(uint16_t, lo[1]) << 16,
-        (uint32_t)__builtin_bit_cast(uint16_t, lo[2]) | (uint32_t)__builtin_bit_cast(uint16_t, lo[3]) << 16);
-    if ((threadIdx.x & 7) == 0) S.dsum[((size_t)t * nsb + sb) * 8 + pos / 32] = s;
+    const unsigned sb = v0 / 256, pos = v0 % 256, sub = pos / 32;
+    uint4* dst = reinterpret_cast<uint4*>(S.xh) + ((size_t)t * nsb + sb) * 64;
+    dst[xh_unit(sub >> 2, odd, (pos & 31) / 8, sub & 3)] = odd ? make_uint4(r0, l0, r1, l1) : make_uint4(h0, r0, h1, r1);
+    if ((threadIdx.x & 7) == 0) {
+      S.dsum[((size_t)t * nsb + sb) * 8 + sub] = s;
+      const float q = s * 0.03125f;   // |s| < 2^20
+      const _Float16 a = (_Float16)q, b = (_Float16)(q - (float)a), c = (_Float16)((q - (float)a) - (float)b);
+      *reinterpret_cast<uint2*>(S.xs + ((size_t)t * nsb + sb) * 32 + 8 * (sub & 3) + 4 * (sub >> 2)) =
+          make_uint2(__builtin_bit_cast(uint16_t, a) | (uint32_t)__builtin_bit_cast(uint16_t, b) << 16,
+                     __builtin_bit_cast(uint16_t, c));
+    }
   }
   if (threadIdx.x == 0) {
     S.dscale[t] = ldexpf(1.f, e);
     if (!ok) flag(S.status, kErrRange);   // a non-finite x makes the token's a and u non-finite
   }
+}
+
+// Nibbles to f16 weights: bits 0..3 and 16..19 of a dword ORed into the f16
+// 1024 are 1024 + q exactly; bits 4..7 and 20..23 are 1024 + 16q. One fused
+// multiply-add by sc and -1024 sc (sc/16 and -64 sc) then leaves sc*q in two
+// halves, exactly (sc*q < 1024): one AND-OR and one packed FMA per two
+// weights, and a shift by 8 per dword for the other four nibbles. (With the
+// FP8 conversion, 2 masks, a shift, 4 conversions and 4 products: 11 against
+// 9 instructions per dword.)
+struct NibScale {
+  f16x2 s, b, s16, b16;
+};
+__device__ __forceinline__ NibScale nib_scale(uint32_t sc) {
+  const _Float16 h = (_Float16)(unsigned short)sc;
+  const f16x2 p = {h, h};
+  NibScale r;
+  r.s = p;
+  r.b = p * (f16x2){(_Float16)-1024.f, (_Float16)-1024.f};
+  r.s16 = p * (f16x2){(_Float16)0.0625f, (_Float16)0.0625f};
+  r.b16 = p * (f16x2){(_Float16)-64.f, (_Float16)-64.f};
+  return r;
+}
+// The masks and the bits of 1024, kept in registers of their own: as literals
+// they would take an AND and an OR (an instruction holds one literal).
+struct NibBits {
+  uint32_t lo, hi, one;
+};
+__device__ __forceinline__ NibBits nib_bits() {
+  NibBits k = {0x000F000Fu, 0x00F000F0u, 0x64006400u};
+  asm("" : "+s"(k.lo));
+  asm("" : "+s"(k.hi));
+  asm("" : "+v"(k.one));
+  return k;
+}
+// sc * the nibbles at bits 4HI and 16 + 4HI of w.
+template <int HI>
+__device__ __forceinline__ uint32_t nib_pair_at(uint32_t w, const NibScale& c, const NibBits& k) {
+  const f16x2 q = __builtin_bit_cast(f16x2, (w & (HI ? k.hi : k.lo)) | k.one);
+  return __builtin_bit_cast(uint32_t, HI ? __builtin_elementwise_fma(q, c.s16, c.b16) : __builtin_elementwise_fma(q, c.s, c.b));
+}
+// The 8 nibbles of w times sc: nibbles 0, 4, 1, 5, 2, 6, 3, 7.
+__device__ __forceinline__ f16x8 nib_octet(uint32_t w, const NibScale& c, const NibBits& k) {
+  const uint32_t w8 = w >> 8;
+  const u32x4 a = {nib_pair_at<0>(w, c, k), nib_pair_at<1>(w, c, k), nib_pair_at<0>(w8, c, k), nib_pair_at<1>(w8, c, k)};
+  return __builtin_bit_cast(f16x8, a);
 }
 
 // LDS bytes per (part, token) row: 512 + 16 of padding, so that the rows of
@@ -4112,20 +4180,275 @@ struct GateUpLds {
 };
 
 
-// Workgroup (tile, slice): wavefront w takes row-block w%4 (gate rows of
+// Gate/up of a tile (one expert, up to 64 of its tokens: MT tiles of 16) on
+// four wavefronts of NB row-blocks each, NB slices per workgroup: wavefront w
+// takes row-blocks NB*w.. of the workgroup's 4 NB (row-block rb: gate rows of
+// neurons 8rb..8rb+7, then their up rows) over the whole row. Weights are the
+// B operand of v_mfma_f32_16x16x32_f16: in the TQ4_KM tiles lane 16kg + i
+// holds sub-block 4p + kg of row i, so B = sc*q (exact in f16, nib_octet) of 8
+// positions of 4 sub-blocks at a time, formed once for all MT tiles, and the
+// super-block's half p is scaled by d once. A = x' in two f16 parts with an
+// accumulator each (a lo product added to the hi sum in the matrix core loses
+// low bits that a neuron's dot, whose main and min terms can nearly cancel,
+// needs), tokens as rows, so that a lane's four results are one weight row's
+// and take that row's d from its own header. The min terms, sum_sub dmin *
+// m_sub * sum(x'_sub), are one more product per super-block: A = the sub-block
+// sums in three f16 parts, B = m (a 6-bit integer).
+//
+// What bounds it: with many tokens per expert the matrix cores, if the
+// operands reach them: an x' operand is read from LDS once per NB products of
+// 16 cycles (at NB = 1 LDS alone would take twice the products' time), a
+// weight is formed once per MT tiles, and a workgroup's NB slices share one
+// copy of the x' that each CU reads from L2 (16 KB per token). With few, the
+// weights' way from memory.
+// x' goes from memory to LDS without passing registers, half a super-block
+// ahead; the weights are requested a super-block ahead into the registers
+// their last use frees.
+// Measured, 20 slices at hidden 4096, against prefill_gate_up_few: 512 tokens
+// 357 (500) us, 4.2 TB/s of weights; 4096 tokens 1155 (2300) us, 0.74 PFLOP/s
+// of f16 products.
+constexpr int kGateUpThreads = 256;
+constexpr int kGateUpHalf = kGateUpTiles * 8 * 1024;   // bytes of x' of half a super-block: [tile][part][v][lane][16 B]
+struct GateUpLds2 {
+  uint8_t x[2][kGateUpHalf];                 // from LDS offset 0: the copies address 64 KB
+  uint8_t xs[2][kGateUpTiles * 1024];        // [super-block parity][tile][lane][16 B] the sums' parts
+};
+// 64 lanes' 16 bytes at rsrc + voff + soff to LDS bytes lds + 16 lane. The
+// compiler does not count this load: a gate_up_wait precedes every use of the
+// bytes, and every load of the compiler's own issued after it.
+__device__ __forceinline__ void lds_copy16(uint32_t lds, uint32_t voff, const u32x4& rsrc, uint32_t soff) {
+  uint32_t m0;
+  asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds\n\ts_mov_b32 m0, %0"
+               : "=&s"(m0)
+               : "s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+// All but the wavefront's last N vector loads are complete, then the
+// workgroup's barrier: every wavefront's copies into LDS are in.
+template <int N>
+__device__ __forceinline__ void gate_up_wait() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int MT, int NB>
+__device__ __forceinline__ void gate_up_tile(const BatchHeader& H, const BatchScratch& S, const BatchTile& T,
+                                             const BatchSlot* slots, unsigned brank0, GateUpLds2& L, uint32_t& bad) {
+  const unsigned nsb = H.hidden / 256, nblk = H.nblk;
+  const int lane = threadIdx.x & 63;
+  const unsigned wave = uniform(threadIdx.x >> 6), kg = (unsigned)lane >> 4, col = (unsigned)lane & 15;
+  const unsigned rank = brank0 + NB * wave / 4, rb0 = NB * wave % 4;
+  // A wavefront past the last slice repeats it and drops the result.
+  const uint64_t slice = H.base[min(rank, nblk - 1)] + (uint64_t)T.expert * H.slice_bytes;
+  const __amdgpu_buffer_rsrc_t W =
+      __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(slice), (short)0, (int)(9216 * nsb), 0x00020000);
+  const uint64_t xa = reinterpret_cast<uint64_t>(S.xh), xn = (uint64_t)H.tokens * nsb * 1024;
+  const u32x4 X = {uniform((uint32_t)xa), uniform((uint32_t)(xa >> 32) & 0xffffu), uniform((uint32_t)xn), 0x00020000u};
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)&L.x[0][0];
+  // Token col of tile m; a tile's missing tokens lie past the buffer's end (no
+  // access, and what LDS then holds only enters their own, unused rows).
+  uint32_t voff[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const unsigned n = 16 * m + col;
+    voff[m] = n < T.ntok ? slots[n].token * (nsb * 1024) + 16 * kg : 0x80000000u;
+  }
+  // Half p of super-block s: wavefront w copies v = w of every (tile, part).
+  auto copy_x = [&](unsigned s, unsigned p) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int part = 0; part < 2; ++part)
+        lds_copy16(lds0 + p * kGateUpHalf + (m * 2 + part) * 4096 + 1024 * wave, voff[m], X,
+                   1024 * s + 16 * xh_unit(p, part, 0, 0) + 64 * wave);
+  };
+  // The sums' parts: wavefront m copies tile m's, through a register (those
+  // past the tile's tokens copy the first token's, which nothing reads).
+  const unsigned sn = 16 * wave + col;
+  const bool sums = sn < T.ntok;
+  const uint8_t* xsrc = reinterpret_cast<const uint8_t*>(S.xs) + (size_t)(sums ? slots[sn].token : 0) * nsb * 64 + 16 * kg;
+  const uint32_t vq = 16 * (uint32_t)lane, vh = 16 * col;
+  auto load_q = [&](unsigned s, unsigned p, u32x4 (&q)[NB]) {
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+      q[n] = __builtin_amdgcn_raw_buffer_load_b128(W, (int)vq, (int)(9216 * s + 1024 + 2048 * (rb0 + n) + 1024 * p), 0);
+  };
+  auto load_h = [&](unsigned s, u32x4 (&h)[NB]) {
+#pragma unroll
+    for (int n = 0; n < NB; ++n) h[n] = __builtin_amdgcn_raw_buffer_load_b128(W, (int)vh, (int)(9216 * s + 256 * (rb0 + n)), 0);
+  };
+  u32x4 q0[NB], q1[NB], h[NB];
+  f32x4 acc[MT][NB];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // Requested a super-block ahead, or half of one where the tiles' products
+  // take long enough and their accumulators need the registers.
+  constexpr bool kFar = MT <= 2;
+  uint4 xs = ld16(xsrc);
+  if (kFar) {
+    load_h(0, h);
+    load_q(0, 0, q0);
+    copy_x(0, 0);
+    load_q(0, 1, q1);
+  } else {
+    copy_x(0, 0);
+    load_h(0, h);
+    load_q(0, 0, q0);
+  }
+  *reinterpret_cast<uint4*>(&L.xs[0][16 * threadIdx.x]) = xs;
+  uint32_t hflag = 0;
+  const NibBits K = nib_bits();
+  // One half super-block's products: buffer p of x', the formed weights. Half
+  // 1 joins the min terms before it joins the sum: one rounding at the sum's
+  // magnitude for both.
+  auto products = [&](int p, unsigned par, const f16x8 (&B)[NB][4], const uint32_t (&dd)[NB], const uint32_t (&sm)[NB]) {
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      __builtin_amdgcn_sched_barrier(0);   // one tile's operands in registers at a time
+      const uint8_t* x = &L.x[p][m * 8192 + 16 * lane];
+      f32x4 ch[NB], cl[NB];
+#pragma unroll
+      for (int n = 0; n < NB; ++n) ch[n] = cl[n] = z;
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const f16x8 xh = *reinterpret_cast<const f16x8*>(x + 1024 * v), xl = *reinterpret_cast<const f16x8*>(x + 4096 + 1024 * v);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          ch[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xh, B[n][v], ch[n], 0, 0, 0);
+          cl[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xl, B[n][v], cl[n], 0, 0, 0);
+        }
+      }
+      if (p == 0) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][n][r] = fmaf(half_to_float(dd[n] & 0xffffu), ch[n][r] + cl[n][r], acc[m][n][r]);
+      } else {
+        // The sums' mid and lo parts in a product of their own.
+        const u32x4 a = *reinterpret_cast<const u32x4*>(&L.xs[par][1024 * m + 16 * lane]);
+        const f16x8 ah = __builtin_bit_cast(f16x8, u32x4{a[0] & 0xffffu, 0u, a[2] & 0xffffu, 0u});
+        const f16x8 al = __builtin_bit_cast(f16x8, u32x4{a[0] & 0xffff0000u, a[1], a[2] & 0xffff0000u, a[3]});
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+          const float d = half_to_float(dd[n] & 0xffffu), dm = -32.f * half_to_float(dd[n] >> 16);   // the sums are over 32
+          const _Float16 m0 = (_Float16)(unsigned short)(sm[n] >> 8 & 0xffu), m1 = (_Float16)(unsigned short)(sm[n] >> 16);
+          const f16x8 b = {m0, m0, m0, m0, m1, m1, m1, m1};
+          f32x4 cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, b, z, 0, 0, 0);
+          cm = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, b, cm, 0, 0, 0);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) acc[m][n][r] += fmaf(dm, cm[r], d * (ch[n][r] + cl[n][r]));
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  for (unsigned s = 0; s < nsb; ++s) {
+    const unsigned sn1 = min(s + 1, nsb - 1), par = s & 1;
+    f16x8 B[NB][4];
+    uint32_t dd[NB], sm[NB];   // d | dmin << 16; sc of sub-block 4 + kg | m of kg << 8 | m of 4 + kg << 16
+    gate_up_wait<kFar ? NB : 2 * NB>();   // x' of half 0; after its copies q1 (near: h, q0) were requested
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      // Sub-blocks kg and 4 + kg of row col (src/native.c:14-19).
+      const uint32_t k = 8 * kg, s0 = h[n][1] >> k, s1 = h[n][2] >> k, s2 = h[n][3] >> k;
+      hflag |= half_bad_bits(h[n][0]);
+      dd[n] = h[n][0];
+      sm[n] = (s2 & 15u) | ((s0 >> 2) & 48u) | (s1 & 63u) << 8 | (((s2 >> 4) & 15u) | ((s1 >> 2) & 48u)) << 16;
+      const NibScale c = nib_scale(s0 & 63u);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) B[n][v] = nib_octet(q0[n][v], c, K);
+    }
+    __builtin_amdgcn_sched_barrier(0);   // the copies follow the waits for h and q0
+    copy_x(s, 1);
+    xs = ld16(xsrc + 64 * (size_t)sn1);
+    if (kFar) {
+      load_q(sn1, 0, q0);
+      load_h(sn1, h);
+    } else {
+      load_q(s, 1, q1);
+    }
+    products(0, par, B, dd, sm);
+    gate_up_wait<kFar ? 2 * NB + 1 : NB + 1>();   // x' of half 1; after its copies: xs, then q0, h (near: q1)
+#pragma unroll
+    for (int n = 0; n < NB; ++n) {
+      const NibScale c = nib_scale(sm[n] & 0xffu);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) B[n][v] = nib_octet(q1[n][v], c, K);
+    }
+    *reinterpret_cast<uint4*>(&L.xs[par ^ 1][16 * threadIdx.x]) = xs;
+    __builtin_amdgcn_sched_barrier(0);   // the copies follow the waits for q1 and xs
+    copy_x(sn1, 0);
+    if (kFar) {
+      load_q(sn1, 1, q1);
+    } else {
+      load_h(sn1, h);
+      load_q(sn1, 0, q0);
+    }
+    products(1, par, B, dd, sm);
+  }
+  gate_up_wait<0>();   // no copy into LDS outlives the workgroup
+  if (hflag & kHalfBadBits) bad |= kErrScale;
+  // Lane (kg, col) holds tokens 4kg..4kg+3 of row col of each row-block: gate
+  // row col or up row col - 8 of neuron 8rb + col%8. The two lanes of a neuron
+  // exchange their values and take two tokens each.
+  if (rank >= nblk) return;
+  const bool up = col >= 8;
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      const unsigned t = 16 * m + 4 * kg + 2 * up + r;
+      const bool in = t < T.ntok;
+      const BatchSlot sl = slots[in ? t : 0];
+      const float sx = S.dscale[sl.token];
+#pragma unroll
+      for (int n = 0; n < NB; ++n) {
+        const float mine = up ? acc[m][n][2 + r] : acc[m][n][r];
+        const float other = dpp_f<kRowRor8>(up ? acc[m][n][r] : acc[m][n][2 + r]);
+        uint32_t hb = 0;
+        const float hv = sl.gate * silu_mul_f32((up ? other : mine) * sx, (up ? mine : other) * sx, hb);
+        if (in) {
+          bad |= hb;
+          S.h[(size_t)(T.slot0 + t) * (nblk * kNeurons) + kNeurons * rank + 8 * (rb0 + n) + (col & 7)] = hv;
+        }
+      }
+    }
+}
+
+template <int NB>
+__global__ __launch_bounds__(kGateUpThreads, 2) void prefill_gate_up(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  // Workgroups go round-robin over the 8 XCDs; a tile's slices go to one XCD,
+  // whose L2 then serves its x', and the tiles (longest first) to each in turn.
+  const unsigned ng = (H.nblk + NB - 1) / NB, b = blockIdx.x, tile = b / 8 / ng * 8 + b % 8, brank0 = NB * (b / 8 % ng);
+  if (tile >= H.ngtiles) return;
+  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.gtiles_off)[tile];
+  const BatchSlot* slots = reinterpret_cast<const BatchSlot*>(plan + H.slots_off) + T.slot0;
+  __shared__ __align__(16) GateUpLds2 L;
+  uint32_t bad = 0;
+  switch ((T.ntok + kTileTokens - 1) / kTileTokens) {
+    case 1: gate_up_tile<1, NB>(H, S, T, slots, brank0, L, bad); break;
+    case 2: gate_up_tile<2, NB>(H, S, T, slots, brank0, L, bad); break;
+    case 3: gate_up_tile<3, NB>(H, S, T, slots, brank0, L, bad); break;
+    default: gate_up_tile<4, NB>(H, S, T, slots, brank0, L, bad); break;
+  }
+  if (bad) flag(S.status, bad);
+}
+
+
+// The same for chunks too small to give every CU its workgroups above: one
+// slice and 16 tokens per workgroup of eight wavefronts. Wavefront w takes row-block w%4 (gate rows of
 // neurons 8rb..8rb+7, then their up rows) and part w/4 (sub-blocks 0-3 or 4-7
-// of every super-block) of the TQ4_KM tiles; lane 16kg + i holds sub-block
-// 4p + kg of row i, which makes it the B operand of v_mfma_f32_16x16x32_f16
-// (column i, k = 8kg..8kg+7) for 8 positions at a time: B = sc*q, exact in
-// f16, so that each MFMA sums over 4 sub-blocks at once and the super-block
-// is scaled by d only once. A = x' in two f16 parts (two MFMAs), tokens as
-// rows, so that the four results of a lane are one weight row's, scaled by
-// that row's d from the lane's own header. The min terms,
-// sum_sub dmin * m_sub * sum(x'_sub), take one fp32 MFMA per super-block; the
-// token's 2^e multiplies a and u at the end. x' moves through LDS one
-// super-block at a time, double-buffered.
-__global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up(const uint8_t* __restrict__ plan,
-                                                                    BatchScratch S) {
+// of every super-block), so that a wavefront's serial run over the row is half
+// as long and an eighth as wide. The min terms take one fp32 MFMA per
+// super-block; x' moves through registers and LDS one super-block at a time,
+// double-buffered.
+__global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_few(const uint8_t* __restrict__ plan,
+                                                                        BatchScratch S) {
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
   // Workgroups go round-robin over the 8 XCDs; each XCD takes a contiguous
   // run of the (tile, slice) list, so that a tile's 20 slices read its x'
@@ -4140,8 +4463,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up(const uint8_
   const unsigned rb = (unsigned)wave & 3, p = (unsigned)wave >> 2, kg = (unsigned)lane >> 4,
                  col = (unsigned)lane & 15;
   __shared__ __align__(16) GateUpLds L;
-  // Staging: thread -> token tl, 32-byte piece c of its 1 KB of x' (part
-  // c/16, positions 16(c%16)..+15).
+  // Staging: thread -> token tl, 32-byte piece c of its 1 KB of x'.
   const unsigned tl = (unsigned)tid >> 5, c = (unsigned)tid & 31;
   const bool live = tl < T.ntok;
   const size_t trow = (size_t)(live ? slots[tl].token : 0) * nsb;
@@ -4163,7 +4485,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up(const uint8_
     }
   };
   auto store_x = [&](unsigned buf, const XStage& X) {
-    uint8_t* row = &L.xh[buf][c / 16][tl][32 * (c % 16)];
+    uint8_t* row = &L.xh[buf][(c >> 3) & 1][tl][256 * (c >> 4) + 32 * (c & 7)];   // units 2c, 2c + 1 (xh_unit)
     *reinterpret_cast<uint4*>(row) = X.d[0];
     *reinterpret_cast<uint4*>(row + 16) = X.d[1];
     if (c < 8) L.xs[buf][tl][c] = X.s;
@@ -4171,6 +4493,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up(const uint8_
   const uint8_t* wq = slice + 1024 + 2048 * rb + 1024 * p + 16 * (unsigned)lane;   // + 9216 s
   const uint8_t* wh = slice + 256 * rb + 16 * col;
   uint32_t bad = 0, hflag = 0;   // hflag: half_bad_bits of the scale words read
+  const NibBits K = nib_bits();
   struct WStage {
     uint4 q, h;
   };
@@ -4194,25 +4517,19 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up(const uint8_
     if (s + 2 < nsb) load_x(s + 2, nxt);
     uint32_t sc, mi;
     q4k_scale_min(hc.y, hc.z, hc.w, 4 * p + kg, sc, mi);
-    const f16x2 sch = f16_pair(sc);
+    const NibScale nsc = nib_scale(sc);
     hflag |= half_bad_bits(hc.x);
     const float d = half_to_float(hc.x & 0xffff);   // of row col, the lane's rows of the product
-    // x' of token col, part h, sub-block 4p + kg at LDS
-    // xh[buf][h][col][2 (32 (4p + kg) + 8v)].
-    const uint8_t* xb8 = &L.xh[buf][0][col][64 * (4 * p + kg)];
+    const uint8_t* xb8 = &L.xh[buf][0][col][256 * p + 16 * kg];   // values 8v.. at + 64v
     // The parts accumulate in tiles of their own: a lo product added to the
     // hi sum in the matrix core loses low bits that a neuron's dot, whose
     // main and min terms can nearly cancel, needs.
     f32x4 c_hi = {0.f, 0.f, 0.f, 0.f}, c_lo = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
-      // Word v: low nibbles = positions 8v..8v+3, high nibbles 8v+4..8v+7.
-      const uint32_t w = word(qc, v), lo = nib_lo(w), hi = nib_hi(w);
-      const u32x4 aw = {nib_pair_sc<false>(lo, sch), nib_pair_sc<true>(lo, sch), nib_pair_sc<false>(hi, sch),
-                        nib_pair_sc<true>(hi, sch)};
-      const f16x8 a = __builtin_bit_cast(f16x8, aw);
-      const uint4 bh = *reinterpret_cast<const uint4*>(xb8 + 16 * v);
-      const uint4 bl = *reinterpret_cast<const uint4*>(xb8 + kTileTokens * kXhRow + 16 * v);
+      const f16x8 a = nib_octet(word(qc, v), nsc, K);
+      const uint4 bh = *reinterpret_cast<const uint4*>(xb8 + 64 * v);
+      const uint4 bl = *reinterpret_cast<const uint4*>(xb8 + kTileTokens * kXhRow + 64 * v);
       c_hi = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bh), a, c_hi, 0, 0, 0);
       c_lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, bl), a, c_lo, 0, 0, 0);
     }
@@ -4617,7 +4934,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
     }
   };
   auto store_x = [&](unsigned buf, const XStage& X) {
-    uint8_t* row = &L.xh[buf][c / 16][tl][32 * (c % 16)];
+    uint8_t* row = &L.xh[buf][(c >> 3) & 1][tl][256 * (c >> 4) + 32 * (c & 7)];   // units 2c, 2c + 1 (xh_unit)
     *reinterpret_cast<uint4*>(row) = X.d[0];
     *reinterpret_cast<uint4*>(row + 16) = X.d[1];
     if (c < 8) L.xs[buf][tl][c] = X.s;
@@ -4654,6 +4971,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
     return W;
   };
   uint32_t bad = 0, hflag = 0;   // hflag: half_bad_bits of the scale words read
+  const NibBits K = nib_bits();
   XStage xa = {{z4, z4}, 0.f}, xb = {{z4, z4}, 0.f};
   load_x(0, xa);
   store_x(0, xa);
@@ -4667,7 +4985,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
     const unsigned buf = s & 1;
     if (s + 2 < nsb) load_x(s + 2, nxt);
     f32x4 c_hi = {0.f, 0.f, 0.f, 0.f}, c_lo = {0.f, 0.f, 0.f, 0.f};
-    f16x2 scs[2][2] = {};
+    NibScale scs[2][2] = {};
     if (kQ4) {
       hflag |= half_bad_bits(W.h.x);
 #pragma unroll
@@ -4676,27 +4994,27 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
         for (int J = 0; J < 2; ++J) {
           uint32_t sc, mi;
           q4k_scale_min(W.h.y, W.h.z, W.h.w, 4 * p + 2 * cc + J, sc, mi);
-          scs[cc][J] = f16_pair(sc);
+          scs[cc][J] = nib_scale(sc);
         }
     }
 #pragma unroll
-    for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-      for (int J = 0; J < 2; ++J) {
+    for (int cc = 0; cc < 2; ++cc) {
+      auto half = [&](auto jj) {
+        constexpr int J = decltype(jj)::value;
         const unsigned sub = 4 * p + 2 * cc + J;   // sub-block of the super-block
+        // Values 8kg.. of the sub-block in x's order: 0, 2, 4, 6, 1, 3, 5, 7.
         u32x4 aw;
         if (kQ4) {
-          const uint32_t w0 = J ? nib_hi(W.q[cc][0].x) : nib_lo(W.q[cc][0].x);
-          const uint32_t w1 = J ? nib_hi(W.q[cc][0].y) : nib_lo(W.q[cc][0].y);
-          aw = u32x4{nib_pair_sc<false>(w0, scs[cc][J]), nib_pair_sc<true>(w0, scs[cc][J]),
-                     nib_pair_sc<false>(w1, scs[cc][J]), nib_pair_sc<true>(w1, scs[cc][J])};
+          const uint2 q = W.q[cc][0];
+          aw = u32x4{nib_pair_at<J>(q.x, scs[cc][J], K), nib_pair_at<J>(q.y, scs[cc][J], K),
+                     nib_pair_at<J>(q.x >> 8, scs[cc][J], K), nib_pair_at<J>(q.y >> 8, scs[cc][J], K)};
         } else {
           const uint2 q = W.q[cc][J];
-          aw = u32x4{int8_pair_f16(q.x, 0x0c010c00u), int8_pair_f16(q.x, 0x0c030c02u), int8_pair_f16(q.y, 0x0c010c00u),
-                     int8_pair_f16(q.y, 0x0c030c02u)};
+          aw = u32x4{int8_pair_f16(q.x, 0x0c020c00u), int8_pair_f16(q.y, 0x0c020c00u), int8_pair_f16(q.x, 0x0c030c01u),
+                     int8_pair_f16(q.y, 0x0c030c01u)};
         }
         const f16x8 a = __builtin_bit_cast(f16x8, aw);
-        const uint8_t* xb8 = &L.xh[buf][0][col][2 * (32 * sub + 8 * kg)];
+        const uint8_t* xb8 = &L.xh[buf][0][col][256 * (sub >> 2) + 64 * kg + 16 * (sub & 3)];
         const uint4 bh = *reinterpret_cast<const uint4*>(xb8);
         const uint4 bl = *reinterpret_cast<const uint4*>(xb8 + kTileTokens * kXhRow);
         if (kQ4) {
@@ -4715,7 +5033,10 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[r] = fmaf(d, ph[r] + pl[r], acc[r]);
         }
-      }
+      };
+      half(std::integral_constant<int, 0>{});
+      half(std::integral_constant<int, 1>{});
+    }
     if (kQ4) {
       const float d = half_to_float(W.h.x & 0xffff);
 #pragma unroll
@@ -5965,11 +6286,40 @@ int fetch_output(hipStream_t s, size_t count, float* y, unsigned* status_out) {
 
 size_t batch_capacity(uint32_t tokens, uint32_t hidden) {
   const size_t slots = (size_t)tokens * 11;
-  return sizeof(BatchHeader) + slots * (sizeof(BatchTile) + sizeof(BatchSlot) + sizeof(uint32_t)) + 4 * 256 +
+  return sizeof(BatchHeader) + slots * (2 * sizeof(BatchTile) + sizeof(BatchSlot) + sizeof(uint32_t)) + 5 * 256 +
          (size_t)tokens * hidden * sizeof(float);
 }
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
+// How prefill_gate_up cuts the routed work: slices per workgroup (NB) and
+// 16-token tiles per workgroup (at most kGateUpTiles), or NB = 0 for
+// prefill_gate_up_few. Four slices per workgroup beat two and one (512 tokens,
+// 20 slices: 363, 430, 591 us; 4096 tokens: 1198, 1469, 2225) unless its last
+// wavefronts have no slice left, and larger tiles form each weight for more
+// tokens; both need about four workgroups per CU (two resident), or the last
+// ones run alone.
+struct GateUpCut {
+  uint32_t nb, cap, tiles;
+};
+GateUpCut gate_up_cut(const std::vector<uint32_t>& count, uint32_t nblk) {
+  uint32_t n[kGateUpTiles + 1] = {};   // workgroup tiles at a cap
+  for (uint32_t c : count)
+    for (uint32_t cap = 1; cap <= (uint32_t)kGateUpTiles; ++cap) n[cap] += (c + kTileTokens * cap - 1) / (kTileTokens * cap);
+  GateUpCut best = {0, 1, n[1]};
+  float least = 0.f;
+  const struct { uint32_t nb; float cost; } kinds[] = {{4, 1.f}, {2, 1.2f}, {1, 1.65f}};
+  for (const auto& k : kinds) {
+    const uint32_t groups = (nblk + k.nb - 1) / k.nb;
+    const float cost = k.cost * (float)(groups * k.nb);
+    if ((best.nb && cost >= least) || n[1] * groups < 4 * E.cus) continue;
+    uint32_t cap = kGateUpTiles;
+    while (cap > 1 && n[cap] * groups < 4 * E.cus) --cap;
+    best = {k.nb, cap, n[cap]};
+    least = cost;
+  }
+  return best;
+}
 
 // Tokens grouped by routed expert (ascending id), each expert's tokens in
 // ascending order, cut into tiles of at most 16, then the tokens with the
@@ -6021,6 +6371,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
     experts += count[id] ? 1u : 0u;
   }
   const uint32_t shtiles = (nshared + kTileTokens - 1) / kTileTokens;
+  const GateUpCut cut = gate_up_cut(count, H->nblk);
   H->hidden = hidden;
   H->tokens = T;
   H->nslots = nslots + nshared;
@@ -6035,7 +6386,10 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
   H->proj = l0->proj;
   H->shared_proj = l0->shared_proj;
   H->tiles_off = (uint32_t)align256(sizeof(BatchHeader));
-  H->slots_off = (uint32_t)align256(H->tiles_off + (size_t)(ntiles + shtiles) * sizeof(BatchTile));
+  H->gtiles_off = (uint32_t)align256(H->tiles_off + (size_t)(ntiles + shtiles) * sizeof(BatchTile));
+  H->ngtiles = cut.tiles;
+  H->gslices = cut.nb;
+  H->slots_off = (uint32_t)align256(H->gtiles_off + (size_t)cut.tiles * sizeof(BatchTile));
   H->tokslot_off = (uint32_t)align256(H->slots_off + (size_t)H->nslots * sizeof(BatchSlot));
   H->x_off = (uint32_t)align256(H->tokslot_off + (size_t)T * 11 * sizeof(uint32_t));
   H->total = H->x_off + T * hidden * (uint32_t)sizeof(float);
@@ -6065,6 +6419,18 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
       B.ntok = count[id] - f < (uint32_t)kTileTokens ? count[id] - f : (uint32_t)kTileTokens;
       B.slot0 = first[id] + f;
       B.pad = 0;
+    }
+  // prefill_gate_up's tiles: an expert's 16-token tiles shared out evenly, the
+  // longest first.
+  BatchTile* gtiles = reinterpret_cast<BatchTile*>(out + H->gtiles_off);
+  for (uint32_t len = cut.cap, g = 0; len > 0; --len)
+    for (int id = 0; id < kRouted; ++id) {
+      const uint32_t nt = (count[id] + kTileTokens - 1) / kTileTokens, n = (nt + cut.cap - 1) / cut.cap;
+      for (uint32_t i = 0; i < n; ++i) {
+        const uint32_t f = kTileTokens * (nt * i / n), end = kTileTokens * (nt * (i + 1) / n);
+        if (end - f != kTileTokens * len) continue;
+        gtiles[g++] = BatchTile{(uint32_t)id, (end < count[id] ? end : count[id]) - f, first[id] + f, 0};
+      }
     }
   for (uint32_t f = 0; f < nshared; f += kTileTokens) {
     BatchTile& B = tiles[k++];
@@ -6105,7 +6471,7 @@ int batch_scratch(const BatchHeader& H) {
     E.bpart_bytes = pb;
     ++E.sample.hot_allocations;
   }
-  const size_t db = (size_t)H.tokens * ((H.hidden / 256) * (1024 + 8 * sizeof(float)) + sizeof(float));
+  const size_t db = (size_t)H.tokens * ((H.hidden / 256) * (1024 + 64 + 8 * sizeof(float)) + sizeof(float));
   if (db > E.bdig_bytes) {
     (void)hipFree(E.bdig);
     E.bdig = nullptr;
@@ -6125,10 +6491,23 @@ int batch_scratch(const BatchHeader& H) {
   return FR_HIP_OK;
 }
 
+// Routed gate/up of all-Q4_K units (gate_up_cut).
+void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchScratch& S, hipStream_t stream) {
+  if (!H.gslices) {
+    hipLaunchKernelGGL(prefill_gate_up_few, dim3(H.ntiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
+    return;
+  }
+  const dim3 g((H.ngtiles + 7) / 8 * 8 * ((H.nblk + H.gslices - 1) / H.gslices)), b(kGateUpThreads);
+  if (H.gslices == 4) hipLaunchKernelGGL(prefill_gate_up<4>, g, b, 0, stream, dev_plan, S);
+  else if (H.gslices == 2) hipLaunchKernelGGL(prefill_gate_up<2>, g, b, 0, stream, dev_plan, S);
+  else hipLaunchKernelGGL(prefill_gate_up<1>, g, b, 0, stream, dev_plan, S);
+}
+
 int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
-      H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens)
+      H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
+      !H.ngtiles || H.ngtiles > H.ntiles || (H.gslices != 0 && H.gslices != 1 && H.gslices != 2 && H.gslices != 4))
     return FR_HIP_INVALID;
   const bool kt = H.gu == TQ4_KM && H.dn == TQ4_KT, nat = H.gu == TQ4_K && H.dn == TMXFP4;
   if (!kt && !nat) return FR_HIP_INVALID;
@@ -6140,7 +6519,8 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   S.y = E.by;
   const size_t nd = (size_t)H.tokens * (H.hidden / 256);
   S.xh = reinterpret_cast<uint16_t*>(E.bdig);
-  S.dsum = reinterpret_cast<float*>(E.bdig + nd * 1024);
+  S.xs = reinterpret_cast<uint16_t*>(E.bdig + nd * 1024);
+  S.dsum = reinterpret_cast<float*>(E.bdig + nd * 1088);
   S.dscale = S.dsum + nd * 8;
   S.status = E.bstatus;
   hipEvent_t* te = E.timing && E.timed < E.timed_cap ? E.tev + 3 * E.timed++ : nullptr;
@@ -6148,7 +6528,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   if (te) CK(hipEventRecord(te[0], stream));
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);
-  if (kt) hipLaunchKernelGGL(prefill_gate_up, dim3(H.ntiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
+  if (kt) launch_gate_up(dev_plan, H, S, stream);
   else
     hipLaunchKernelGGL(prefill_gate_up_rows<TQ4_K>, dim3(H.ntiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan,
                        S, 0u);
