@@ -4036,6 +4036,7 @@ static_assert(sizeof(BatchHeader) == 264, "batch header layout");
 constexpr uint32_t kNoSlot = ~0u;        // tokslot entry of a token without the shared expert
 struct BatchScratch {
   float* h;                              // [nslots][nblk * 32] gate * h
+  uint32_t* hmax;                        // [nslots] bits of the largest |gate * h| (prefill_down)
   float* part;                           // [nslots][hidden] per-(token, expert) partials
   float* y;                              // [tokens][hidden]
   uint16_t* xh;                          // [tokens][super-block][512] x' = x * 2^-e as f16 hi, lo (xh_unit)
@@ -4068,6 +4069,7 @@ __global__ __launch_bounds__(1024) void prefill_split(const uint8_t* __restrict_
   __shared__ float red[16];
   __shared__ uint32_t nonfinite;
   if (threadIdx.x == 0) nonfinite = 0;
+  if (threadIdx.x < 11 && 11 * t + threadIdx.x < H.nslots) S.hmax[11 * t + threadIdx.x] = 0;
   float m = fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)));
   const bool fin = isfinite(x.x) && isfinite(x.y) && isfinite(x.z) && isfinite(x.w);
 #pragma unroll
@@ -4132,15 +4134,17 @@ __global__ __launch_bounds__(1024) void prefill_split(const uint8_t* __restrict_
 struct NibScale {
   f16x2 s, b, s16, b16;
 };
-__device__ __forceinline__ NibScale nib_scale(uint32_t sc) {
-  const _Float16 h = (_Float16)(unsigned short)sc;
-  const f16x2 p = {h, h};
+__device__ __forceinline__ NibScale nib_scales(f16x2 p) {   // scales of the low and the high half's nibbles
   NibScale r;
   r.s = p;
   r.b = p * (f16x2){(_Float16)-1024.f, (_Float16)-1024.f};
   r.s16 = p * (f16x2){(_Float16)0.0625f, (_Float16)0.0625f};
   r.b16 = p * (f16x2){(_Float16)-64.f, (_Float16)-64.f};
   return r;
+}
+__device__ __forceinline__ NibScale nib_scale(uint32_t sc) {
+  const _Float16 h = (_Float16)(unsigned short)sc;
+  return nib_scales((f16x2){h, h});
 }
 // The masks and the bits of 1024, kept in registers of their own: as literals
 // they would take an AND and an OR (an instruction holds one literal).
@@ -4405,17 +4409,24 @@ __device__ __forceinline__ void gate_up_tile(const BatchHeader& H, const BatchSc
       const bool in = t < T.ntok;
       const BatchSlot sl = slots[in ? t : 0];
       const float sx = S.dscale[sl.token];
+      float top = 0.f;
 #pragma unroll
       for (int n = 0; n < NB; ++n) {
         const float mine = up ? acc[m][n][2 + r] : acc[m][n][r];
         const float other = dpp_f<kRowRor8>(up ? acc[m][n][r] : acc[m][n][2 + r]);
         uint32_t hb = 0;
         const float hv = sl.gate * silu_mul_f32((up ? other : mine) * sx, (up ? mine : other) * sx, hb);
+        top = fmaxf(top, fabsf(hv));
         if (in) {
           bad |= hb;
           S.h[(size_t)(T.slot0 + t) * (nblk * kNeurons) + kNeurons * rank + 8 * (rb0 + n) + (col & 7)] = hv;
         }
       }
+      // The token's largest |h| over the wavefront's neurons.
+      top = fmaxf(top, dpp_f<kQuadXor1>(top));
+      top = fmaxf(top, dpp_f<kQuadXor2>(top));
+      top = fmaxf(top, dpp_f<kRowHalfMirror>(top));
+      if (in && (col & 7) == 0) atomicMax(S.hmax + T.slot0 + t, __float_as_uint(top));
     }
 }
 
@@ -4595,6 +4606,326 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
   }
 }
 
+// Down of a tile (one expert, up to 64 of its tokens: MT tiles of 16) onto the
+// 256 outputs of one super-block, over all owned slices: four wavefronts of 64
+// outputs (four 16-output tiles) each. With the Q4_K-T down's weight w = d sc q
+// - dmin m (src/native.c:14-22; per neuron n a super-block over the outputs,
+// sub-block g of 32 outputs), a slice adds
+//   sum_n d_n sc_ng q_on h'_n  -  sum_n dmin_n m_ng h'_n
+// to output o of sub-block g, with h' = h * 2^-e_t (per token t, e_t puts the
+// largest |h'| of the token's slices in [2^12, 2^13)). Both sums run on
+// v_mfma_f32_16x16x32_f16 over the 32 neurons (lane group kq: 8kq..8kq+7):
+//   A[o][n] = sc_ng * q_on exactly in f16 (sc q < 1024), formed once for all MT
+//     tiles of tokens. A lane's 16-byte unit holds 4 outputs x 8 neurons, dword
+//     w neurons 2w (nibbles 0..3: the outputs) and 2w + 1 (4..7); tile t takes
+//     output t of every unit, so that a tile's operand lies in the lane's own
+//     unit, two neurons to a nib_pair_at;
+//   B[n][t] = d_n h'_nt in two f16 parts (22 significant bits). It serves all
+//     256 outputs, so one wavefront forms it for the four, through LDS: with
+//     MTP (MT up to a power of two) token tiles a round takes RS = 4/MTP
+//     slices, wavefront w forms (slice w/MTP, token tile w%MTP);
+//   the min terms' A[g][n] = m_ng, B = dmin_n h'_nt in two parts, by the same
+//     wavefront, eight of sixteen rows in use.
+// The products add straight into the accumulators over the slices. The rounds
+// are pipelined behind one barrier each: while round i's products run, round
+// i+1's B is formed and the scales of round i+2 are unpacked.
+// A slice in which a neuron's |d| or |dmin| is 4 or more (d h' could leave
+// f16's range; no real unit has one) contributes nothing in the rounds and is
+// taken at the end with B scaled down by a power of two.
+//
+// What bounds it: the vector units, busy 0.7 of the time (A, B and the tables:
+// 350 instructions per four slices with 16 tokens, 160 per slice with 64),
+// with the matrix units' 0.2 (0.35) beside them; four workgroups per CU (a
+// fourth is worth 12 % even at the price of a few spilled registers with 64
+// tokens). Measured, 20 slices at hidden 4096, against prefill_down_few:
+// 512 tokens 200 (215) us, 4096 tokens 730 (1100) us.
+constexpr float kDownDirect = 4.f;
+constexpr int kDownThreads = 256, kDownWaves = kDownThreads / 64;
+struct DownLds {
+  // [round mod 3][slice of the round]
+  _Float16 sc[3][4][8][kNeurons];            // 6-bit scale of (sub-block, neuron)
+  _Float16 mn[3][4][8][kNeurons];            // 6-bit min
+  float d[3][4][kNeurons], dm[3][4][kNeurons];
+  uint4 b[2][kDownWaves][2][64];             // [round mod 2][slice, token tile][part][lane]: B
+  float corr[kDownWaves][8][kTileTokens];    // each wavefront's min terms [sub-block][token]
+  uint32_t deferred;                         // slices with a large d or dmin (bit R)
+};
+
+// v as two f16 values hi = f16(v), lo = f16(v - hi) (v - hi is exact in fp32).
+// v is opaque to the compiler: a v that is a product would otherwise be
+// rounded to f16 straight from the exact product (v_fma_mixlo_f16) in one use
+// of hi and by way of fp32 in the other, and where the two roundings differ
+// hi + lo is off by 2^-11 of v (one super-block of y by up to 8e-5, measured).
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_f16(const float (&v)[8], f16x8& hi, f16x8& lo) {
+  u32x4 h, l;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    float x = v[2 * j], y = v[2 * j + 1];
+    asm("" : "+v"(x));
+    asm("" : "+v"(y));
+    const f16x2 p = __builtin_convertvector((f32x2){x, y}, f16x2);
+    h[j] = __builtin_bit_cast(uint32_t, p);
+    l[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2){fmaf((float)p[0], -1.f, x), fmaf((float)p[1], -1.f, y)}, f16x2));
+  }
+  hi = __builtin_bit_cast(f16x8, h);
+  lo = __builtin_bit_cast(f16x8, l);
+}
+// e_t of a slot from the bits of its largest |gate * h|.
+__device__ __forceinline__ int down_exponent(uint32_t hmax) {
+  int E = 0;
+  if (hmax) (void)frexpf(__uint_as_float(hmax), &E);   // |h| < 2^E
+  return max(E - 13, -126);                            // 2^-e_t is a float
+}
+
+template <int MT>
+__device__ __forceinline__ void down_tile(const BatchHeader& H, const BatchScratch& S, const BatchTile& T, unsigned sb,
+                                          DownLds& L, uint32_t& bad) {
+  constexpr unsigned MTP = MT == 3 ? 4 : MT, RS = 4 / MTP;
+  const unsigned hidden = H.hidden, nblk = H.nblk, nh = nblk * kNeurons, rounds = (nblk + RS - 1) / RS;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const unsigned wave = uniform((unsigned)tid >> 6);
+  const unsigned col = (unsigned)lane & 15, kq = (unsigned)lane >> 4;
+  const unsigned wm = wave % MTP, wr = wave / MTP;   // the token tile and slice the wavefront forms
+  const uint64_t eoff = (uint64_t)T.expert * H.slice_bytes + 2 * H.proj + 4608 * (uint64_t)sb;
+  const uint32_t vu = 1024 * kq + 16 * (16 * wave + col);
+  const unsigned og = 2 * wave + (col >> 3);   // sub-block of the lane's outputs 64 wave + 4 col + 0..3
+  const NibBits K = nib_bits();
+  const unsigned hn = (unsigned)tid & 31;   // neuron whose header the thread unpacks
+  const unsigned fslot = T.slot0 + min(16 * wm + col, T.ntok - 1);
+  const float* hsrc = S.h + (size_t)fslot * nh + 8 * kq;
+  const float fscale = ldexpf(1.f, -down_exponent(S.hmax[fslot]));   // 2^-e_t
+  uint32_t hflag = 0;   // half_bad_bits of the scale words read
+  auto rsrc = [&](unsigned R) {
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(H.base[min(R, nblk - 1)] + eoff), (short)0, 4608,
+                                             0x00020000);
+  };
+  auto load_units = [&](unsigned i, u32x4 (&U)[RS]) {
+#pragma unroll
+    for (unsigned r = 0; r < RS; ++r) U[r] = __builtin_amdgcn_raw_buffer_load_b128(rsrc(RS * i + r), (int)vu, 0, 0);
+  };
+  auto load_header = [&](unsigned R) {
+    return u32x4(__builtin_amdgcn_raw_buffer_load_b128(rsrc(R), (int)(4096 + 16 * hn), 0, 0));
+  };
+  struct HRow {
+    float4 a, b;
+  };
+  auto load_h = [&](unsigned R) {
+    const float4* p = reinterpret_cast<const float4*>(hsrc + kNeurons * min(R, nblk - 1));
+    return HRow{p[0], p[1]};
+  };
+  // Scales of sub-blocks g0..g0+n-1 of the thread's neuron into table (buf, r).
+  auto unpack = [&](const u32x4& hd, unsigned buf, unsigned r, unsigned g0, unsigned n) {
+    hflag |= half_bad_bits(hd[0]);
+#pragma unroll
+    for (unsigned i = 0; i < n; ++i) {
+      uint32_t sc, mi;
+      q4k_scale_min(hd[1], hd[2], hd[3], g0 + i, sc, mi);
+      L.sc[buf][r][g0 + i][hn] = (_Float16)(unsigned short)sc;
+      L.mn[buf][r][g0 + i][hn] = (_Float16)(unsigned short)mi;
+    }
+    if (g0 == 0) {
+      L.d[buf][r][hn] = half_to_float(hd[0] & 0xffffu);
+      L.dm[buf][r][hn] = half_to_float(hd[0] >> 16);
+    }
+  };
+  // 256/RS threads per slice, RS sub-blocks each.
+  const unsigned g0 = ((unsigned)tid % (kDownThreads / RS) >> 5) * RS;
+  auto table = [&](unsigned i, unsigned buf, const u32x4& hd) {
+    const unsigned R = RS * i + wr;
+    unpack(hd, buf, wr, g0, RS);
+    const bool large = !(fabsf(half_to_float(hd[0] & 0xffffu)) < kDownDirect) || !(fabsf(half_to_float(hd[0] >> 16)) < kDownDirect);
+    if (__builtin_expect(__ballot(large) != 0 && R < nblk, 0)) atomicOr(&L.deferred, 1u << R);
+  };
+  f32x4 acc[MT][4], cmin = {0.f, 0.f, 0.f, 0.f};
+  const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[m][q] = z;
+  // The wavefront's B of table (buf, r) times 2^-k, into bo; the min terms.
+  auto form = [&](const HRow& hr, bool live, unsigned buf, unsigned r, int k, uint4* bo) {
+    const float4* dp = reinterpret_cast<const float4*>(&L.d[buf][r][8 * kq]);
+    const float4* mp = reinterpret_cast<const float4*>(&L.dm[buf][r][8 * kq]);
+    const float4 d0 = dp[0], d1 = dp[1], m0 = mp[0], m1 = mp[1];
+    const float hv[8] = {hr.a.x, hr.a.y, hr.a.z, hr.a.w, hr.b.x, hr.b.y, hr.b.z, hr.b.w};
+    const float dv[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
+    const float mv[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+    float v[8], w[8];
+    const float f = live ? fscale : 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float hs = hv[j] * f;   // exact
+      v[j] = k ? ldexpf(hs * dv[j], -k) : hs * dv[j];
+      w[j] = k ? ldexpf(hs * mv[j], -k) : hs * mv[j];
+    }
+    f16x8 hi, lo;
+    split_f16(v, hi, lo);
+    bo[lane] = __builtin_bit_cast(uint4, hi);
+    bo[64 + lane] = __builtin_bit_cast(uint4, lo);
+    split_f16(w, hi, lo);
+    const f16x8 a = *reinterpret_cast<const f16x8*>(&L.mn[buf][r][col & 7][8 * kq]);
+    f32x4 c = k ? z : cmin;
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, lo, c, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, hi, c, 0, 0, 0);
+    if (k) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) cmin[j] += ldexpf(c[j], k);
+    } else {
+      cmin = c;
+    }
+  };
+  // A of the wavefront's four output tiles from the lane's unit, table (buf, r).
+  auto a_tiles = [&](const u32x4& U, unsigned buf, unsigned r, f16x8 (&a)[4]) {
+    const u32x4 s4 = *reinterpret_cast<const u32x4*>(&L.sc[buf][r][og][8 * kq]);
+    u32x4 t[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      const uint32_t sp = s4[w], x = U[w], x8 = x >> 8;
+      const NibScale c = nib_scales(__builtin_bit_cast(f16x2, sp));
+      t[0][w] = nib_pair_at<0>(x, c, K);
+      t[1][w] = nib_pair_at<1>(x, c, K);
+      t[2][w] = nib_pair_at<0>(x8, c, K);
+      t[3][w] = nib_pair_at<1>(x8, c, K);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) a[q] = __builtin_bit_cast(f16x8, t[q]);
+  };
+  auto products = [&](unsigned i, unsigned buf, const u32x4 (&U)[RS]) {
+#pragma unroll
+    for (unsigned r = 0; r < RS; ++r) {
+      if (r && RS * i + r >= nblk) break;
+      f16x8 a[4];
+      a_tiles(U[r], buf, r, a);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const f16x8 bh = __builtin_bit_cast(f16x8, L.b[i & 1][r * MTP + m][0][lane]);
+        const f16x8 bl = __builtin_bit_cast(f16x8, L.b[i & 1][r * MTP + m][1][lane]);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[q], bl, acc[m][q], 0, 0, 0);
+          acc[m][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[q], bh, acc[m][q], 0, 0, 0);
+        }
+      }
+    }
+  };
+  auto direct = [&](unsigned R) { return R < nblk && !(L.deferred >> R & 1u); };
+  u32x4 ua[RS], ub[RS];
+  // The first rounds' bytes all at once: one trip to memory.
+  u32x4 ha = load_header(wr), hb = load_header(RS + wr);
+  HRow hr = load_h(wr);
+  load_units(0, ua);
+  u32x4 hc = load_header(2 * RS + wr), hd = load_header(3 * RS + wr);
+  HRow hr1 = load_h(RS + wr);
+  load_units(1, ub);
+  if (tid == 0) L.deferred = 0;
+  __syncthreads();   // deferred is cleared
+  table(0, 0, ha);
+  table(1, 1, hb);
+  __syncthreads();
+  form(hr, direct(wr), 0, wr, 0, &L.b[0][wave][0][0]);
+  hr = hr1;
+  __syncthreads();
+  // Round i's products beside round i+1's B and round i+2's scales (past the
+  // last round: the last slice's, B as zero). Units and headers are requested
+  // two rounds before their use, h (in L2) one.
+  unsigned t0 = 0, t1 = 1, t2 = 2;
+  auto round = [&](unsigned i, u32x4 (&U)[RS], u32x4& head) {
+    const unsigned R = RS * (i + 1) + wr;
+    form(hr, direct(R), t1, wr, 0, &L.b[(i + 1) & 1][wave][0][0]);
+    hr = load_h(R + RS);
+    table(i + 2, t2, head);
+    head = load_header(R + 3 * RS);
+    products(i, t0, U);
+    load_units(i + 2, U);
+    __syncthreads();
+    const unsigned t = t0;
+    t0 = t1;
+    t1 = t2;
+    t2 = t;
+  };
+  for (unsigned i = 0; i < rounds; i += 2) {
+    round(i, ua, hc);
+    if (i + 1 < rounds) round(i + 1, ub, hd);
+  }
+  // Deferred slices: B = d h' 2^-k with 2^k >= max(|d|, |dmin|) / 4 over the
+  // slice's neurons, each product times 2^k before it joins the sum.
+  for (uint32_t dfr = L.deferred; dfr; dfr &= dfr - 1) {
+    const unsigned R = (unsigned)__builtin_ctz(dfr);
+    const u32x4 hw = load_header(R), U = __builtin_amdgcn_raw_buffer_load_b128(rsrc(R), (int)vu, 0, 0);
+    const HRow h1 = load_h(R);
+    unpack(hw, 0, 0, (unsigned)tid >> 5, 1);
+    float dmax = fmaxf(fabsf(half_to_float(hw[0] & 0xffffu)), fabsf(half_to_float(hw[0] >> 16)));
+    dmax = isfinite(dmax) ? dmax : 0.f;   // a non-finite scale is flagged
+#pragma unroll
+    for (int o = 16; o; o >>= 1) dmax = fmaxf(dmax, __shfl_xor(dmax, o));
+    int E = 0;
+    (void)frexpf(dmax, &E);   // dmax < 2^E
+    const int k = max(E - 2, 1);
+    __syncthreads();   // the slice's table is in
+    if (wave < MT) form(h1, true, 0, 0, k, &L.b[0][wave][0][0]);
+    __syncthreads();   // and its B
+    f16x8 a[4];
+    a_tiles(U, 0, 0, a);
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        f32x4 pr = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[q], __builtin_bit_cast(f16x8, L.b[0][m][1][lane]), z, 0, 0, 0);
+        pr = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[q], __builtin_bit_cast(f16x8, L.b[0][m][0][lane]), pr, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[m][q][r] += ldexpf(pr[r], k);
+      }
+    __syncthreads();   // the table and B are read before the next deferred slice writes them
+  }
+  // The min terms of sub-block g and token col: rows 4kq + j of each
+  // wavefront's product, summed over the wavefronts of a token tile.
+  if (kq < 2)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) L.corr[wave][4 * kq + j][col] = cmin[j];
+  __syncthreads();
+  if (hflag & kHalfBadBits) bad |= kErrScale;
+  // Lane (kq, col) holds rows 4kq + r of every tile q for token col: outputs 64
+  // wave + 4(4kq + r) + q. y = (C - min terms) * 2^e_t.
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    if (16 * m + col >= T.ntok) continue;
+    const unsigned slot = T.slot0 + 16 * m + col;
+    const int et = down_exponent(S.hmax[slot]);
+    float* dst = S.part + (size_t)slot * hidden + 256 * sb + 64 * wave + 16 * kq;
+    float c = 0.f;
+#pragma unroll
+    for (unsigned r = 0; r < RS; ++r) c += L.corr[r * MTP + m][2 * wave + (kq >> 1)][col];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      *reinterpret_cast<float4*>(dst + 4 * r) =
+          make_float4(ldexpf(acc[m][0][r] - c, et), ldexpf(acc[m][1][r] - c, et), ldexpf(acc[m][2][r] - c, et),
+                      ldexpf(acc[m][3][r] - c, et));
+  }
+}
+
+__global__ __launch_bounds__(kDownThreads, 4) void prefill_down(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  // A tile's super-blocks on one XCD, whose L2 serves its h; the tiles
+  // (longest first) to each XCD in turn.
+  const unsigned nsb = H.hidden / 256, b = blockIdx.x, tile = b / 8 / nsb * 8 + b % 8, sb = b / 8 % nsb;
+  if (tile >= H.ngtiles) return;
+  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.gtiles_off)[tile];
+  __shared__ __align__(16) DownLds L;
+  uint32_t bad = 0;
+  switch ((T.ntok + kTileTokens - 1) / kTileTokens) {
+    case 1: down_tile<1>(H, S, T, sb, L, bad); break;
+    case 2: down_tile<2>(H, S, T, sb, L, bad); break;
+    case 3: down_tile<3>(H, S, T, sb, L, bad); break;
+    default: down_tile<4>(H, S, T, sb, L, bad); break;
+  }
+  if (bad) flag(S.status, bad);
+}
+
+// The down of chunks that prefill_gate_up_few takes (16-token tiles): each
+// wavefront forms B for itself and needs no barrier, which is the better
+// bargain for few slices (64 tokens, one slice, hidden 4096: the whole launch
+// 54 us, 66 us with prefill_down; 200 tokens, seven slices: 202 and 207 us).
 // Workgroup (tile, 512 outputs), four wavefronts: wavefront w takes the 128
 // outputs 256 sb + 128 hb .. +127 (sb = 2 blockIdx.y + w/2, hb = w%2), eight
 // 16-output tiles in one pass over all owned slices (B, the slice's header
@@ -4618,12 +4949,11 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
 // in which a neuron's |d| is 4 or more (d h' could leave f16's range; no real
 // unit has such a d) is deferred to the end and taken with B scaled down by
 // a power of two.
-constexpr float kDownDirect = 4.f;
-// prefill_down's workgroups: 4 wavefronts over 512 outputs (two super-blocks),
-// three workgroups per CU (168 registers per lane: the eight tiles' accumulators
-// and two slices of bytes in flight).
-constexpr int kDownThreads = 256, kDownWaves = kDownThreads / 64, kDownWgCols = 512;
-struct DownLds {
+// The workgroups take 512 outputs (two super-blocks), three of them per CU (168
+// registers per lane: the eight tiles' accumulators and two slices of bytes in
+// flight).
+constexpr int kDownFewCols = 512;
+struct DownFewLds {
   float h[kBlocks][4][kTileTokens][8];   // [slice][round q][token][neuron 8q + i]: gate * h * 2^-e_t
   int e[kTileTokens];                    // e_t
   // [wave][slice parity][sub-block 4hb + j of the wavefront][neuron]
@@ -4632,27 +4962,12 @@ struct DownLds {
   float d[kDownWaves][2][kNeurons];          // d
 };
 
-// v as two f16 values hi = f16(v), lo = f16(v - hi) (v - hi is exact in fp32).
-// v is opaque to the compiler: a v that is a product would otherwise be
-// rounded to f16 straight from the exact product (v_fma_mixlo_f16) in one use
-// of hi and by way of fp32 in the other, and where the two roundings differ
-// hi + lo is off by 2^-11 of v (one super-block of y by up to 8e-5, measured).
-__device__ __forceinline__ void split_f16(const float (&v)[8], f16x8& hi, f16x8& lo) {
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    float x = v[j];
-    asm("" : "+v"(x));
-    hi[j] = (_Float16)x;
-    lo[j] = (_Float16)(x - (float)hi[j]);
-  }
-}
-
-__global__ __launch_bounds__(kDownThreads, 3) void prefill_down(const uint8_t* __restrict__ plan, BatchScratch S) {
+__global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_t* __restrict__ plan, BatchScratch S) {
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
   const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.tiles_off)[blockIdx.x];
   const unsigned hidden = H.hidden, nsb = hidden / 256, nblk = H.nblk;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  __shared__ __align__(16) DownLds L;
+  __shared__ __align__(16) DownFewLds L;
   const unsigned nh = nblk * kNeurons;
 #pragma unroll 1
   for (unsigned th = 0; th < kTileTokens / (kDownThreads / 32); ++th) {
@@ -6452,7 +6767,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
 // Scratch of the prefill kernels, grown on demand (never inside a timed
 // region once warm: the sizes depend only on the token count).
 int batch_scratch(const BatchHeader& H) {
-  const size_t hb = (size_t)H.nslots * H.nblk * kNeurons * sizeof(float);
+  const size_t hb = (size_t)H.nslots * (H.nblk * kNeurons * sizeof(float) + sizeof(uint32_t));   // h, then hmax
   const size_t pb = (size_t)H.nslots * H.hidden * sizeof(float);
   const size_t yb = (size_t)H.tokens * H.hidden * sizeof(float);
   if (hb > E.bh_bytes) {
@@ -6515,6 +6830,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   if (rc) return rc;
   BatchScratch S;
   S.h = E.bh;
+  S.hmax = reinterpret_cast<uint32_t*>(E.bh + (size_t)H.nslots * H.nblk * kNeurons);
   S.part = E.bpart;
   S.y = E.by;
   const size_t nd = (size_t)H.tokens * (H.hidden / 256);
@@ -6537,9 +6853,12 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
                        dev_plan, S, H.ntiles);
   const unsigned ncol_mx = (H.hidden + down_rows_cols<TMXFP4>() - 1) / down_rows_cols<TMXFP4>();
   const unsigned ncol_q8 = (H.hidden + down_rows_cols<TQ8_0>() - 1) / down_rows_cols<TQ8_0>();
-  if (kt)
-    hipLaunchKernelGGL(prefill_down, dim3(H.ntiles, (H.hidden + kDownWgCols - 1) / kDownWgCols), dim3(kDownThreads), 0,
-                       stream, dev_plan, S);
+  if (kt && H.gslices)
+    hipLaunchKernelGGL(prefill_down, dim3((H.ngtiles + 7) / 8 * 8 * (H.hidden / 256)), dim3(kDownThreads), 0, stream,
+                       dev_plan, S);
+  else if (kt)
+    hipLaunchKernelGGL(prefill_down_few, dim3(H.ntiles, (H.hidden + kDownFewCols - 1) / kDownFewCols),
+                       dim3(kDownThreads), 0, stream, dev_plan, S);
   else
     hipLaunchKernelGGL(prefill_down_rows<TMXFP4>, dim3(H.ntiles, ncol_mx), dim3(kBatchThreads), 0, stream, dev_plan,
                        S, 0u);
