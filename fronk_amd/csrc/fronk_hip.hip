@@ -5207,15 +5207,26 @@ __device__ __forceinline__ uint32_t int8_pair_f16(uint32_t v, uint32_t sel) {
   return __builtin_bit_cast(uint32_t, f);
 }
 
-template <int GU>
-__global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const uint8_t* __restrict__ plan,
-                                                                         BatchScratch S, uint32_t tile0) {
+// LDS of the rows' gate/up. Q4_K rows, two super-blocks at a time: [row][half]
+// [8 chunks][16 B] (a row padded to 272 bytes, so that the 16 rows a read
+// spans fall in different banks) and [row][super-block][16 B] headers; filled
+// from registers loaded one stage ahead, each row half read as one 128-byte
+// run.
+constexpr unsigned kRowPad = 272;
+template <bool Q4>
+struct GateUpRowsLds {
+  GateUpLds x;
+  uint8_t wq[Q4 ? 64 * kRowPad : 16];
+  uint4 wh[Q4 ? 64 * 2 : 1];
+};
+// One (tile, slice).
+template <int GU, class Lds>
+__device__ __forceinline__ void gate_up_rows_tile(const uint8_t* __restrict__ plan, const BatchScratch& S, unsigned tile,
+                                                  unsigned brank, Lds& LL) {
   constexpr bool kQ4 = GU == TQ4_K;
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
-  // XCD-contiguous runs of the (tile, slice) list, as prefill_gate_up.
-  const unsigned nblk = H.nblk, per = gridDim.x / 8, b = blockIdx.x;
-  const unsigned j = b < 8 * per ? (b % 8) * per + b / 8 : b, brank = j % nblk;
-  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.tiles_off)[tile0 + j / nblk];
+  const unsigned nblk = H.nblk;
+  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.tiles_off)[tile];
   const BatchSlot* slots = reinterpret_cast<const BatchSlot*>(plan + H.slots_off) + T.slot0;
   const unsigned hidden = H.hidden, nsb = hidden / 256, nch = hidden / 64;
   const uint64_t proj = kQ4 ? H.proj : H.shared_proj;
@@ -5223,15 +5234,10 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned rb = (unsigned)wave & 3, p = (unsigned)wave >> 2, kg = (unsigned)lane >> 4,
                  col = (unsigned)lane & 15, i = col;
-  __shared__ __align__(16) GateUpLds L;
-  // Q4_K rows, two super-blocks at a time: [row][half][8 chunks][16 B] (a row
-  // padded to 272 bytes, so that the 16 rows a read spans fall in different
-  // banks) and [row][super-block][16 B] headers; filled from registers loaded
-  // one stage ahead, each row half read as one 128-byte run.
-  constexpr unsigned kRowPad = 272;
-  __shared__ __align__(16) uint8_t WQ[kQ4 ? 64 * kRowPad : 16];
-  __shared__ __align__(16) uint4 WH[kQ4 ? 64 * 2 : 1];
-  // x' staging, as prefill_gate_up: thread -> token tl, 32-byte piece c.
+  GateUpLds& L = LL.x;
+  uint8_t* WQ = LL.wq;
+  uint4* WH = LL.wh;
+  // x' staging, as prefill_gate_up_few: thread -> token tl, 32-byte piece c.
   const unsigned tl = (unsigned)tid >> 5, c = (unsigned)tid & 31;
   const bool live = tl < T.ntok;
   const size_t trow = (size_t)(live ? slots[tl].token : 0) * nsb;
@@ -5467,6 +5473,31 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const u
   if (bad) flag(S.status, bad);
 }
 
+// The native chunk's gate/up, shared expert's tiles (the longer ones) first and
+// the routed tiles in the same launch: the shared expert's alone are too few
+// to fill the chip (37 tokens, 7 slices: a launch of its own takes 19 us beside
+// the routed one's 43 us).
+__global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  __shared__ __align__(16) GateUpRowsLds<true> L;
+  const unsigned nblk = H.nblk, ns = H.shtiles * nblk;
+  if (blockIdx.x < ns) {
+    gate_up_rows_tile<TQ8_0>(plan, S, H.ntiles + blockIdx.x / nblk, blockIdx.x % nblk, L);
+    return;
+  }
+  // XCD-contiguous runs of the (tile, slice) list: a tile's slices read its x'
+  // from one L2.
+  const unsigned per = (gridDim.x - ns) / 8, b = blockIdx.x - ns, j = b < 8 * per ? (b % 8) * per + b / 8 : b;
+  gate_up_rows_tile<TQ4_K>(plan, S, j / nblk, j % nblk, L);
+}
+// The shared expert's alone (beside all-Q4_K units).
+__global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_shared(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  __shared__ __align__(16) GateUpRowsLds<false> L;
+  const unsigned per = gridDim.x / 8, b = blockIdx.x, j = b < 8 * per ? (b % 8) * per + b / 8 : b;
+  gate_up_rows_tile<TQ8_0>(plan, S, H.ntiles + j / H.nblk, j % H.nblk, L);
+}
+
 // Down (tile, 128 kT outputs) of row-format units: output o's 32 neurons as
 // one record (MXFP4: 16 code bytes at 16o, neuron j in the low nibble of byte
 // j, 16 + j in its high nibble, E8M0 exponent at 16H + o; Q8_0: 16 int8 at
@@ -5498,19 +5529,16 @@ constexpr unsigned down_rows_cols() {
 struct DownRowsLds {
   bf16x8 b[kBlocks][3][64];   // [slice][part][lane 16kq + token m]: k-slots 2i, 2i+1 = neurons 4kq + i, 16 + 4kq + i
 };
-// The Q8_0 instantiation holds twice the record bytes per tile and takes two
-// wavefronts per SIMD instead of four.
+// One (tile, column group).
 template <int DN>
-__global__ __launch_bounds__(kBatchThreads, DN == TMXFP4 ? 4 : 2) void prefill_down_rows(const uint8_t* __restrict__ plan,
-                                                                                          BatchScratch S,
-                                                                                          uint32_t tile0) {
+__device__ __forceinline__ void down_rows_tile(const uint8_t* __restrict__ plan, const BatchScratch& S, unsigned tile,
+                                               unsigned group, DownRowsLds& L) {
   constexpr bool kMx = DN == TMXFP4;
   constexpr int kT = kMx ? kDownRowsTilesMx : kDownRowsTilesQ8;
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
-  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.tiles_off)[tile0 + blockIdx.x];
+  const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.tiles_off)[tile];
   const unsigned hidden = H.hidden, nblk = H.nblk;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  __shared__ __align__(16) DownRowsLds L;
   const unsigned nh = nblk * kNeurons;
   // Item (slice R, lane 16kq + n): token n's gate * h of neurons 4kq..4kq+3
   // and 16 + 4kq..+3, interleaved into the lane's k-slots, in three parts.
@@ -5530,7 +5558,7 @@ __global__ __launch_bounds__(kBatchThreads, DN == TMXFP4 ? 4 : 2) void prefill_d
     L.b[R][2][ln] = b3;
   }
   __syncthreads();
-  const unsigned o0 = down_rows_cols<DN>() * blockIdx.y + 16 * kT * (unsigned)wave;
+  const unsigned o0 = down_rows_cols<DN>() * group + 16 * kT * (unsigned)wave;
   if (o0 >= hidden) return;
   const unsigned m = (unsigned)lane & 15, kq = (unsigned)lane >> 4;
   const uint64_t proj = kMx ? H.proj : H.shared_proj;
@@ -5691,6 +5719,23 @@ __global__ __launch_bounds__(kBatchThreads, DN == TMXFP4 ? 4 : 2) void prefill_d
       *reinterpret_cast<float4*>(dst + 16 * t) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
   }
   if (bad) flag(S.status, bad);
+}
+
+// The native chunk's down, the shared expert's tiles first (as
+// prefill_gate_up_rows).
+__global__ __launch_bounds__(kBatchThreads, 4) void prefill_down_rows(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  __shared__ __align__(16) DownRowsLds L;
+  const unsigned ns = H.shtiles * ((H.hidden + down_rows_cols<TQ8_0>() - 1) / down_rows_cols<TQ8_0>()), b = blockIdx.x;
+  if (b < ns) down_rows_tile<TQ8_0>(plan, S, H.ntiles + b % H.shtiles, b / H.shtiles, L);
+  else down_rows_tile<TMXFP4>(plan, S, (b - ns) % H.ntiles, (b - ns) / H.ntiles, L);
+}
+// The shared expert's alone: it holds twice the record bytes per tile and takes
+// two wavefronts per SIMD instead of four.
+__global__ __launch_bounds__(kBatchThreads, 2) void prefill_down_shared(const uint8_t* __restrict__ plan, BatchScratch S) {
+  const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
+  __shared__ __align__(16) DownRowsLds L;
+  down_rows_tile<TQ8_0>(plan, S, H.ntiles + blockIdx.x % H.shtiles, blockIdx.x / H.shtiles, L);
 }
 
 // Token t's outputs 1024 by..+1023: its 10 expert partials in routing order,
@@ -6844,27 +6889,25 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   if (te) CK(hipEventRecord(te[0], stream));
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);
-  if (kt) launch_gate_up(dev_plan, H, S, stream);
-  else
-    hipLaunchKernelGGL(prefill_gate_up_rows<TQ4_K>, dim3(H.ntiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan,
-                       S, 0u);
-  if (H.shtiles)
-    hipLaunchKernelGGL(prefill_gate_up_rows<TQ8_0>, dim3(H.shtiles * H.nblk), dim3(kBatchThreads), 0, stream,
-                       dev_plan, S, H.ntiles);
-  const unsigned ncol_mx = (H.hidden + down_rows_cols<TMXFP4>() - 1) / down_rows_cols<TMXFP4>();
-  const unsigned ncol_q8 = (H.hidden + down_rows_cols<TQ8_0>() - 1) / down_rows_cols<TQ8_0>();
-  if (kt && H.gslices)
-    hipLaunchKernelGGL(prefill_down, dim3((H.ngtiles + 7) / 8 * 8 * (H.hidden / 256)), dim3(kDownThreads), 0, stream,
+  const unsigned down_q8 = H.shtiles * ((H.hidden + down_rows_cols<TQ8_0>() - 1) / down_rows_cols<TQ8_0>());
+  if (kt) {
+    launch_gate_up(dev_plan, H, S, stream);
+    if (H.shtiles)
+      hipLaunchKernelGGL(prefill_gate_up_shared, dim3(H.shtiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
+    if (H.gslices)
+      hipLaunchKernelGGL(prefill_down, dim3((H.ngtiles + 7) / 8 * 8 * (H.hidden / 256)), dim3(kDownThreads), 0, stream,
+                         dev_plan, S);
+    else
+      hipLaunchKernelGGL(prefill_down_few, dim3(H.ntiles, (H.hidden + kDownFewCols - 1) / kDownFewCols),
+                         dim3(kDownThreads), 0, stream, dev_plan, S);
+    if (H.shtiles)
+      hipLaunchKernelGGL(prefill_down_shared, dim3(down_q8), dim3(kBatchThreads), 0, stream, dev_plan, S);
+  } else {
+    const unsigned down_mx = H.ntiles * ((H.hidden + down_rows_cols<TMXFP4>() - 1) / down_rows_cols<TMXFP4>());
+    hipLaunchKernelGGL(prefill_gate_up_rows, dim3((H.shtiles + H.ntiles) * H.nblk), dim3(kBatchThreads), 0, stream,
                        dev_plan, S);
-  else if (kt)
-    hipLaunchKernelGGL(prefill_down_few, dim3(H.ntiles, (H.hidden + kDownFewCols - 1) / kDownFewCols),
-                       dim3(kDownThreads), 0, stream, dev_plan, S);
-  else
-    hipLaunchKernelGGL(prefill_down_rows<TMXFP4>, dim3(H.ntiles, ncol_mx), dim3(kBatchThreads), 0, stream, dev_plan,
-                       S, 0u);
-  if (H.shtiles)
-    hipLaunchKernelGGL(prefill_down_rows<TQ8_0>, dim3(H.shtiles, ncol_q8), dim3(kBatchThreads), 0, stream, dev_plan,
-                       S, H.ntiles);
+    hipLaunchKernelGGL(prefill_down_rows, dim3(down_q8 + down_mx), dim3(kBatchThreads), 0, stream, dev_plan, S);
+  }
   if (te) CK(hipEventRecord(te[1], stream));
   hipLaunchKernelGGL(prefill_reduce, dim3(H.tokens, ncol), dim3(256), 0, stream, dev_plan, S);
   if (te) CK(hipEventRecord(te[2], stream));
