@@ -4011,7 +4011,9 @@ __global__ void synth_kernel(uint8_t* __restrict__ dst, SliceShape routed, Slice
 constexpr int kTileTokens = 16;          // tokens of one expert tile (the MFMA N)
 constexpr int kBatchThreads = 512;
 constexpr int kMaxBatchTokens = 4096;
-constexpr int kDownCols = 1024;          // outputs of one prefill_down workgroup
+constexpr int kDownCols = 1024;          // outputs of one prefill_reduce workgroup
+constexpr size_t kBatchPiece = 512 * 1024;   // bytes of x and y on their way at a time (fr_hip_run_batch)
+constexpr size_t kBatchStaged = 1024 * 1024; // plans up to this size travel by kernel
 
 constexpr int kGateUpTiles = 4;          // 16-token tiles of one prefill_gate_up workgroup at most
 
@@ -6091,9 +6093,13 @@ struct Engine {
   uint8_t* bdig = nullptr;            // x' parts, then sub-block sums, then 2^e
   size_t bh_bytes = 0, bpart_bytes = 0, by_bytes = 0, bdig_bytes = 0;
   uint32_t* bstatus = nullptr;
+  uint32_t* blast = nullptr;          // the last batch launch's status word (bstatus or bplan_dev's)
   uint32_t* bstatus_host = nullptr;   // pinned
   uint8_t* bplan_dev = nullptr;
   uint8_t* bplan_host = nullptr;      // pinned
+  float* by_host = nullptr;           // pinned: fr_hip_run_batch's y
+  size_t by_host_bytes = 0;
+  hipEvent_t bpiece[2] = {};          // its pieces on their way to by_host
   size_t bplan_cap = 0;
   uint32_t batch_tokens = 0, batch_hidden = 0;
 };
@@ -6554,6 +6560,15 @@ __global__ __launch_bounds__(64) void stage_plan(const uint4* __restrict__ src, 
   if (i < words) dst[i] = src[i];
 }
 
+// The way back: `words` 16-byte words and one status word into mapped pinned
+// host memory.
+__global__ __launch_bounds__(64) void stage_out(const uint4* __restrict__ src, uint4* __restrict__ dst, unsigned words,
+                                                const uint32_t* __restrict__ status, uint32_t* __restrict__ dstatus) {
+  const unsigned i = blockIdx.x * 64 + threadIdx.x;
+  if (i < words) dst[i] = src[i];
+  if (i == 0) *dstatus = *status;
+}
+
 // `host`: a decode plan's y and status words go to the engine's mapped host
 // buffers (fr_hip_run), and the engine's output parity is left as it is.
 int launch(const uint8_t* dev_plan, const PlanHeader& H, unsigned grid, hipStream_t stream, bool host = false) {
@@ -6688,8 +6703,9 @@ GateUpCut gate_up_cut(const std::vector<uint32_t>& count, uint32_t nblk) {
 // order in which its partials are summed (backends/ref.c:61-97). Every
 // loaded block has one format: Q4_K-T units (routed on prefill_gate_up /
 // prefill_down) or native units (Q4_K rows, MXFP4 down: the row-format
-// prefill kernels); the shared expert is Q8_0 in both.
-int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
+// prefill kernels); the shared expert is Q8_0 in both. Without `with_x` the
+// x of the plan is left for the caller to fill in.
+int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used, bool with_x = true) {
   if (!r || !out || !used || !r->expert || !r->gate || !r->x) return FR_HIP_INVALID;
   if (!r->tokens || r->tokens > (unsigned)kMaxBatchTokens || r->layer >= (unsigned)kLayers || r->mode > MODE_Q8_256)
     return FR_HIP_INVALID;
@@ -6799,7 +6815,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used) {
     B.slot0 = nslots + f;
     B.pad = 0;
   }
-  memcpy(out + H->x_off, r->x, (size_t)T * hidden * sizeof(float));
+  if (with_x) memcpy(out + H->x_off, r->x, (size_t)T * hidden * sizeof(float));
   *used = H->total;
   E.sample.unique_experts = experts;
   E.sample.pairs = ntiles * H->nblk;
@@ -6863,7 +6879,9 @@ void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchSc
   else hipLaunchKernelGGL(prefill_gate_up<1>, g, b, 0, stream, dev_plan, S);
 }
 
-int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream) {
+// `status`: a device word that the stream has zeroed by then, or null for the
+// engine's.
+int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream, uint32_t* status = nullptr) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
       H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
@@ -6883,9 +6901,9 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   S.xs = reinterpret_cast<uint16_t*>(E.bdig + nd * 1024);
   S.dsum = reinterpret_cast<float*>(E.bdig + nd * 1088);
   S.dscale = S.dsum + nd * 8;
-  S.status = E.bstatus;
+  S.status = E.blast = status ? status : E.bstatus;
   hipEvent_t* te = E.timing && E.timed < E.timed_cap ? E.tev + 3 * E.timed++ : nullptr;
-  CK(hipMemsetAsync(E.bstatus, 0, sizeof(uint32_t), stream));
+  if (!status) CK(hipMemsetAsync(E.bstatus, 0, sizeof(uint32_t), stream));
   if (te) CK(hipEventRecord(te[0], stream));
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);
@@ -6920,7 +6938,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
 int batch_output(hipStream_t s, float* y, size_t count, unsigned* status_out) {
   if (count > (size_t)E.batch_tokens * E.batch_hidden) return FR_HIP_INVALID;
   uint32_t status = 0;
-  CK(hipMemcpyAsync(E.bstatus_host, E.bstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  CK(hipMemcpyAsync(E.bstatus_host, E.blast ? E.blast : E.bstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   CK(hipStreamSynchronize(s));
   status = *E.bstatus_host;
   if (status_out) *status_out = status;
@@ -7034,11 +7052,12 @@ static int open_engine(int device) {
   CK(hipHostMalloc(reinterpret_cast<void**>(&E.out_host), (size_t)E.out_words * sizeof(uint32_t), hipHostMallocDefault));
   CK(hipMalloc(&E.bstatus, sizeof(uint32_t)));
   CK(hipMemset(E.bstatus, 0, sizeof(uint32_t)));
-  CK(hipHostMalloc(reinterpret_cast<void**>(&E.bstatus_host), sizeof(uint32_t), hipHostMallocDefault));
+  CK(hipHostMalloc(reinterpret_cast<void**>(&E.bstatus_host), sizeof(uint32_t), hipHostMallocMapped));
   CK(hipEventCreate(&E.ev0));
   CK(hipEventCreate(&E.ev1));
   CK(hipEventCreate(&E.pev0));
   CK(hipEventCreate(&E.pev1));
+  for (hipEvent_t& e : E.bpiece) CK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   CK(hipDeviceSynchronize());
   g_open = true;
   return FR_HIP_OK;
@@ -7076,6 +7095,9 @@ void release_engine() {
   (void)hipFree(E.bstatus);
   (void)hipFree(E.bplan_dev);
   (void)hipHostFree(E.bplan_host);
+  (void)hipHostFree(E.by_host);
+  for (hipEvent_t e : E.bpiece)
+    if (e) (void)hipEventDestroy(e);
   (void)hipHostFree(E.bstatus_host);
   (void)hipHostFree(E.plan_host);
   (void)hipHostFree(E.out_host);
@@ -7393,35 +7415,104 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
   if (!req || !y) return FR_HIP_INVALID;
   CK(hipSetDevice(E.device));
   if (req->tokens > (unsigned)kMaxBatchTokens) return FR_HIP_INVALID;
-  const size_t need = batch_capacity(req->tokens, req->hidden);
+  const size_t need = ((batch_capacity(req->tokens, req->hidden) + 15) & ~size_t(15)) + 16;   // the status word follows the plan
   if (need > E.bplan_cap) {
     (void)hipFree(E.bplan_dev);
     (void)hipHostFree(E.bplan_host);
     E.bplan_dev = nullptr;
     E.bplan_host = nullptr;
     E.bplan_cap = 0;
+    E.blast = nullptr;
     CK(hipMalloc(&E.bplan_dev, need));
-    CK(hipHostMalloc(reinterpret_cast<void**>(&E.bplan_host), need, hipHostMallocDefault));
+    CK(hipHostMalloc(reinterpret_cast<void**>(&E.bplan_host), need, hipHostMallocMapped));
     E.bplan_cap = need;
   }
   size_t used = 0;
-  int rc = build_batch(req, E.bplan_host, E.bplan_cap, &used);
+  int rc = build_batch(req, E.bplan_host, E.bplan_cap - 16, &used, false);
   if (rc) return rc;
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(E.bplan_host);
-  CK(hipMemcpyAsync(E.bplan_dev, E.bplan_host, used, hipMemcpyHostToDevice, E.stream));
+  const size_t bytes = (size_t)H.tokens * H.hidden * sizeof(float);
+  if (bytes > E.by_host_bytes) {
+    (void)hipHostFree(E.by_host);
+    E.by_host = nullptr;
+    E.by_host_bytes = 0;
+    CK(hipHostMalloc(reinterpret_cast<void**>(&E.by_host), bytes, hipHostMallocMapped));
+    E.by_host_bytes = bytes;
+  }
+  // The plan, x and a zero status word go up, y and the status come back through
+  // pinned memory of the engine; y goes to the caller once the status is known.
+  // Small plans travel by copy kernels, whose start costs less than a DMA
+  // engine's (37 tokens, hidden 2560: 150 us per call by DMA, 7 us of them per
+  // copy and 45 us between the copies and the kernels). Larger ones
+  // travel in pieces, each on its way while the host copies the next
+  // (512 tokens: 1058 us per call with one copy each way, 1020 us in pieces).
+  const bool staged = used <= kBatchStaged;
+  const uint32_t zero = 0;
+  if (staged) {
+    memcpy(E.bplan_host + H.x_off, req->x, bytes);
+    memcpy(E.bplan_host + used, &zero, sizeof(zero));
+    void* mapped = nullptr;
+    CK(hipHostGetDevicePointer(&mapped, E.bplan_host, 0));
+    const unsigned words = (unsigned)((used + sizeof(zero) + 15) / 16);
+    hipLaunchKernelGGL(stage_plan, dim3((words + 63) / 64), dim3(64), 0, E.stream, static_cast<const uint4*>(mapped),
+                       reinterpret_cast<uint4*>(E.bplan_dev), words);
+  }
+  for (size_t at = 0, end = used + sizeof(zero); !staged && at < end;) {
+    const size_t next = at ? at + kBatchPiece : H.x_off + kBatchPiece, to = next + kBatchPiece / 2 < end ? next : end;
+    const size_t x0 = at > H.x_off ? at : H.x_off, x1 = to < used ? to : used;
+    if (x1 > x0)
+      memcpy(E.bplan_host + x0, reinterpret_cast<const uint8_t*>(req->x) + (x0 - H.x_off), x1 - x0);
+    if (to == end) memcpy(E.bplan_host + used, &zero, sizeof(zero));
+    CK(hipMemcpyAsync(E.bplan_dev + at, E.bplan_host + at, to - at, hipMemcpyHostToDevice, E.stream));
+    at = to;
+  }
   CK(hipEventRecord(E.ev0, E.stream));
-  rc = batch_launch(E.bplan_dev, H, E.stream);
+  uint32_t* dstatus = reinterpret_cast<uint32_t*>(E.bplan_dev + used);
+  rc = batch_launch(E.bplan_dev, H, E.stream, dstatus);
   if (rc) return rc;
   CK(hipEventRecord(E.ev1, E.stream));
-  unsigned status = 0;
-  rc = batch_output(E.stream, nullptr, 0, &status);
-  if (rc) return rc;
+  if (staged) {
+    void *my = nullptr, *ms = nullptr;
+    CK(hipHostGetDevicePointer(&my, E.by_host, 0));
+    CK(hipHostGetDevicePointer(&ms, E.bstatus_host, 0));
+    const unsigned words = (unsigned)(bytes / 16);
+    hipLaunchKernelGGL(stage_out, dim3((words + 63) / 64), dim3(64), 0, E.stream, reinterpret_cast<const uint4*>(E.by),
+                       static_cast<uint4*>(my), words, dstatus, static_cast<uint32_t*>(ms));
+    CK(hipStreamSynchronize(E.stream));
+  } else {
+    CK(hipMemcpyAsync(E.bstatus_host, dstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, E.stream));
+  }
+  auto fetch = [&](size_t k) {   // piece k of y, if there is one
+    const size_t at = k * kBatchPiece;
+    if (at >= bytes) return hipSuccess;
+    const hipError_t e = hipMemcpyAsync(reinterpret_cast<uint8_t*>(E.by_host) + at, reinterpret_cast<uint8_t*>(E.by) + at,
+                                        bytes - at < kBatchPiece ? bytes - at : kBatchPiece, hipMemcpyDeviceToHost, E.stream);
+    return e == hipSuccess ? hipEventRecord(E.bpiece[k & 1], E.stream) : e;
+  };
+  if (!staged) {
+    CK(fetch(0));
+    CK(fetch(1));
+    CK(hipEventSynchronize(E.bpiece[0]));
+  }
+  const unsigned status = *E.bstatus_host;
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, E.ev0, E.ev1) == hipSuccess) E.sample.last_kernel_ns = ms * 1e6;
   ++E.sample.runs;
-  if (status) return FR_HIP_NUMERIC;
-  // y is written only on success: untouched on failure.
-  CK(hipMemcpy(y, E.by, (size_t)H.tokens * H.hidden * sizeof(float), hipMemcpyDeviceToHost));
+  if (status) {
+    CK(hipStreamSynchronize(E.stream));
+    return FR_HIP_NUMERIC;   // y is written only on success: untouched on failure
+  }
+  if (staged) {
+    memcpy(y, E.by_host, bytes);
+    return FR_HIP_OK;
+  }
+  for (size_t k = 0; k * kBatchPiece < bytes; ++k) {
+    const size_t at = k * kBatchPiece;
+    if (k) CK(hipEventSynchronize(E.bpiece[k & 1]));
+    CK(fetch(k + 2));
+    memcpy(reinterpret_cast<uint8_t*>(y) + at, reinterpret_cast<uint8_t*>(E.by_host) + at,
+           bytes - at < kBatchPiece ? bytes - at : kBatchPiece);
+  }
   return FR_HIP_OK;
 }
 

@@ -262,3 +262,29 @@ def test_prefill_gate_up_cuts(eng, hidden, nblk, tokens, pool, slices):
     rows = rng.choice(tokens, 7, replace=False)
     ref = oracle_rows(lay, blocks, 0, experts[rows], gates[rows], x[rows])
     check_close(ref, y[rows], fa.MODE_F32, ("cut", hidden, nblk))
+
+
+@pytest.mark.parametrize("tokens", [1, 60, 63, 64, 130, 300])
+def test_prefill_run_batch_equals_resident_plan(eng, tokens):
+    """fr_hip_run_batch's way up and down (copy kernels up to 1 MB of plan, which
+    64 tokens at hidden 4096 pass; 512 KB pieces above) leaves y what a resident
+    plan gives, bit for bit; and after a call that fails, fr_hip_batch_output
+    reports that call's status."""
+    import ctypes as C
+
+    import torch
+    hidden = 4096
+    load(eng, hidden, (0, 7))
+    rng = np.random.default_rng(tokens)
+    experts, gates, x = chunk(rng, tokens, hidden)
+    y = run_ok(eng, 0, experts, gates, x)
+    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+    dev = torch.from_numpy(plan).to("cuda")
+    torch.cuda.synchronize()
+    ref, status = np.zeros_like(x), C.c_uint()
+    assert fa.lib().fr_hip_batch_launch(plan.ctypes.data, dev.data_ptr(), None) == fa.OK
+    assert fa.lib().fr_hip_batch_output(None, fa.fptr(ref), x.size, C.byref(status)) == fa.OK
+    assert status.value == 0 and np.array_equal(y.view(np.uint32), ref.view(np.uint32))
+    x[-1, -1] = np.inf
+    assert eng.run_batch(0, experts, gates, x)[0] == fa.NUMERIC
+    assert fa.lib().fr_hip_batch_output(None, None, 0, C.byref(status)) == fa.OK and status.value != 0
