@@ -6867,6 +6867,10 @@ int batch_scratch(const BatchHeader& H) {
   return FR_HIP_OK;
 }
 
+// Zeroes a status word. A kernel because a caller may capture the launch: a
+// memset node in a graph has given wrong results on replays after the first.
+__global__ void clear_word(uint32_t* w) { *w = 0; }
+
 // Routed gate/up of all-Q4_K units (gate_up_cut).
 void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchScratch& S, hipStream_t stream) {
   if (!H.gslices) {
@@ -6903,7 +6907,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   S.dscale = S.dsum + nd * 8;
   S.status = E.blast = status ? status : E.bstatus;
   hipEvent_t* te = E.timing && E.timed < E.timed_cap ? E.tev + 3 * E.timed++ : nullptr;
-  if (!status) CK(hipMemsetAsync(E.bstatus, 0, sizeof(uint32_t), stream));
+  if (!status) hipLaunchKernelGGL(clear_word, dim3(1), dim3(1), 0, stream, E.bstatus);
   if (te) CK(hipEventRecord(te[0], stream));
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);

@@ -288,3 +288,32 @@ def test_prefill_run_batch_equals_resident_plan(eng, tokens):
     x[-1, -1] = np.inf
     assert eng.run_batch(0, experts, gates, x)[0] == fa.NUMERIC
     assert fa.lib().fr_hip_batch_output(None, None, 0, C.byref(status)) == fa.OK and status.value != 0
+
+
+def test_prefill_captured_launch_records_kernels_only(eng):
+    """A captured fr_hip_batch_launch holds kernel nodes alone: a memset node has
+    given wrong results on replays after the first."""
+    import ctypes as C
+
+    import torch
+    hidden = 4096
+    load(eng, hidden, (0, 7))
+    rng = np.random.default_rng(9)
+    experts, gates, x = chunk(rng, 40, hidden)
+    run_ok(eng, 0, experts, gates, x)   # the scratch is grown before the capture
+    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+    dev = torch.from_numpy(plan).to("cuda")
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+        assert fa.lib().fr_hip_batch_launch(plan.ctypes.data, dev.data_ptr(), C.c_void_p(s.cuda_stream)) == fa.OK
+    with open("/proc/self/maps") as f:
+        hip = C.CDLL(next(line.split()[-1] for line in f if "libamdhip64" in line))
+    graph, n = C.c_void_p(g.raw_cuda_graph()), C.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value
+    nodes = (C.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+    for node in nodes:
+        kind = C.c_int()
+        assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
+        assert kind.value == 0, kind.value   # hipGraphNodeTypeKernel
