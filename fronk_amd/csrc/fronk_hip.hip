@@ -6093,7 +6093,6 @@ struct Engine {
   uint8_t* bdig = nullptr;            // x' parts, then sub-block sums, then 2^e
   size_t bh_bytes = 0, bpart_bytes = 0, by_bytes = 0, bdig_bytes = 0;
   uint32_t* bstatus = nullptr;
-  uint32_t* blast = nullptr;          // the last batch launch's status word (bstatus or bplan_dev's)
   uint32_t* bstatus_host = nullptr;   // pinned
   uint8_t* bplan_dev = nullptr;
   uint8_t* bplan_host = nullptr;      // pinned
@@ -6553,11 +6552,13 @@ bool launch_decode(const uint8_t* dev_plan, const PlanHeader& H, unsigned grid, 
 // Copies a plan from mapped pinned host memory into device memory, one
 // 16-byte word per lane with every load in flight at once: one PCIe round
 // trip, where a DMA copy first waits for its engine and then for the kernels'
-// queue (about 4 us more per run, measured).
+// queue (about 4 us more per run, measured). `clear`: a status word to zero on
+// the way, or null.
 __global__ __launch_bounds__(64) void stage_plan(const uint4* __restrict__ src, uint4* __restrict__ dst,
-                                                 unsigned words) {
+                                                 unsigned words, uint32_t* __restrict__ clear) {
   const unsigned i = blockIdx.x * 64 + threadIdx.x;
   if (i < words) dst[i] = src[i];
+  if (clear && i == 0) *clear = 0;
 }
 
 // The way back: `words` 16-byte words and one status word into mapped pinned
@@ -6883,9 +6884,8 @@ void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchSc
   else hipLaunchKernelGGL(prefill_gate_up<1>, g, b, 0, stream, dev_plan, S);
 }
 
-// `status`: a device word that the stream has zeroed by then, or null for the
-// engine's.
-int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream, uint32_t* status = nullptr) {
+// `cleared`: the stream has zeroed the status word by then.
+int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream, bool cleared = false) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
       H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
@@ -6905,9 +6905,9 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   S.xs = reinterpret_cast<uint16_t*>(E.bdig + nd * 1024);
   S.dsum = reinterpret_cast<float*>(E.bdig + nd * 1088);
   S.dscale = S.dsum + nd * 8;
-  S.status = E.blast = status ? status : E.bstatus;
+  S.status = E.bstatus;
   hipEvent_t* te = E.timing && E.timed < E.timed_cap ? E.tev + 3 * E.timed++ : nullptr;
-  if (!status) hipLaunchKernelGGL(clear_word, dim3(1), dim3(1), 0, stream, E.bstatus);
+  if (!cleared) hipLaunchKernelGGL(clear_word, dim3(1), dim3(1), 0, stream, E.bstatus);
   if (te) CK(hipEventRecord(te[0], stream));
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);
@@ -6942,7 +6942,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
 int batch_output(hipStream_t s, float* y, size_t count, unsigned* status_out) {
   if (count > (size_t)E.batch_tokens * E.batch_hidden) return FR_HIP_INVALID;
   uint32_t status = 0;
-  CK(hipMemcpyAsync(E.bstatus_host, E.blast ? E.blast : E.bstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+  CK(hipMemcpyAsync(E.bstatus_host, E.bstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   CK(hipStreamSynchronize(s));
   status = *E.bstatus_host;
   if (status_out) *status_out = status;
@@ -7343,7 +7343,7 @@ int run_once(const fr_hip_request* req, float* y, bool layer, unsigned* status_o
   {
     const unsigned words = (unsigned)((used + 15) / 16);
     hipLaunchKernelGGL(stage_plan, dim3((words + 63) / 64), dim3(64), 0, E.stream, E.plan_mapped,
-                       reinterpret_cast<uint4*>(E.plan_dev), words);
+                       reinterpret_cast<uint4*>(E.plan_dev), words, static_cast<uint32_t*>(nullptr));
   }
   const bool decode = H.kind == KIND_DECODE || H.kind == KIND_DECODE_ROWS || H.kind == KIND_DECODE_SPLIT ||
                       H.kind == KIND_DECODE_BURST;
@@ -7419,20 +7419,19 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
   if (!req || !y) return FR_HIP_INVALID;
   CK(hipSetDevice(E.device));
   if (req->tokens > (unsigned)kMaxBatchTokens) return FR_HIP_INVALID;
-  const size_t need = ((batch_capacity(req->tokens, req->hidden) + 15) & ~size_t(15)) + 16;   // the status word follows the plan
+  const size_t need = (batch_capacity(req->tokens, req->hidden) + 15) & ~size_t(15);   // copied in 16-byte words
   if (need > E.bplan_cap) {
     (void)hipFree(E.bplan_dev);
     (void)hipHostFree(E.bplan_host);
     E.bplan_dev = nullptr;
     E.bplan_host = nullptr;
     E.bplan_cap = 0;
-    E.blast = nullptr;
     CK(hipMalloc(&E.bplan_dev, need));
     CK(hipHostMalloc(reinterpret_cast<void**>(&E.bplan_host), need, hipHostMallocMapped));
     E.bplan_cap = need;
   }
   size_t used = 0;
-  int rc = build_batch(req, E.bplan_host, E.bplan_cap - 16, &used, false);
+  int rc = build_batch(req, E.bplan_host, E.bplan_cap, &used, false);
   if (rc) return rc;
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(E.bplan_host);
   const size_t bytes = (size_t)H.tokens * H.hidden * sizeof(float);
@@ -7443,36 +7442,35 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
     CK(hipHostMalloc(reinterpret_cast<void**>(&E.by_host), bytes, hipHostMallocMapped));
     E.by_host_bytes = bytes;
   }
-  // The plan, x and a zero status word go up, y and the status come back through
-  // pinned memory of the engine; y goes to the caller once the status is known.
+  // The plan with x goes up, y and the status come back through pinned memory of
+  // the engine; y goes to the caller once the status is known. The status is
+  // the engine's word, as in every batch launch, and is zeroed on the way up.
   // Small plans travel by copy kernels, whose start costs less than a DMA
   // engine's (37 tokens, hidden 2560: 150 us per call by DMA, 7 us of them per
   // copy and 45 us between the copies and the kernels). Larger ones
   // travel in pieces, each on its way while the host copies the next
   // (512 tokens: 1058 us per call with one copy each way, 1020 us in pieces).
   const bool staged = used <= kBatchStaged;
-  const uint32_t zero = 0;
   if (staged) {
     memcpy(E.bplan_host + H.x_off, req->x, bytes);
-    memcpy(E.bplan_host + used, &zero, sizeof(zero));
     void* mapped = nullptr;
     CK(hipHostGetDevicePointer(&mapped, E.bplan_host, 0));
-    const unsigned words = (unsigned)((used + sizeof(zero) + 15) / 16);
+    const unsigned words = (unsigned)((used + 15) / 16);
     hipLaunchKernelGGL(stage_plan, dim3((words + 63) / 64), dim3(64), 0, E.stream, static_cast<const uint4*>(mapped),
-                       reinterpret_cast<uint4*>(E.bplan_dev), words);
+                       reinterpret_cast<uint4*>(E.bplan_dev), words, E.bstatus);
+  } else {
+    hipLaunchKernelGGL(clear_word, dim3(1), dim3(1), 0, E.stream, E.bstatus);
   }
-  for (size_t at = 0, end = used + sizeof(zero); !staged && at < end;) {
-    const size_t next = at ? at + kBatchPiece : H.x_off + kBatchPiece, to = next + kBatchPiece / 2 < end ? next : end;
-    const size_t x0 = at > H.x_off ? at : H.x_off, x1 = to < used ? to : used;
-    if (x1 > x0)
-      memcpy(E.bplan_host + x0, reinterpret_cast<const uint8_t*>(req->x) + (x0 - H.x_off), x1 - x0);
-    if (to == end) memcpy(E.bplan_host + used, &zero, sizeof(zero));
+  for (size_t at = 0; !staged && at < used;) {
+    const size_t next = at ? at + kBatchPiece : H.x_off + kBatchPiece, to = next + kBatchPiece / 2 < used ? next : used;
+    const size_t x0 = at > H.x_off ? at : H.x_off;
+    if (to > x0)
+      memcpy(E.bplan_host + x0, reinterpret_cast<const uint8_t*>(req->x) + (x0 - H.x_off), to - x0);
     CK(hipMemcpyAsync(E.bplan_dev + at, E.bplan_host + at, to - at, hipMemcpyHostToDevice, E.stream));
     at = to;
   }
   CK(hipEventRecord(E.ev0, E.stream));
-  uint32_t* dstatus = reinterpret_cast<uint32_t*>(E.bplan_dev + used);
-  rc = batch_launch(E.bplan_dev, H, E.stream, dstatus);
+  rc = batch_launch(E.bplan_dev, H, E.stream, true);
   if (rc) return rc;
   CK(hipEventRecord(E.ev1, E.stream));
   if (staged) {
@@ -7481,10 +7479,10 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
     CK(hipHostGetDevicePointer(&ms, E.bstatus_host, 0));
     const unsigned words = (unsigned)(bytes / 16);
     hipLaunchKernelGGL(stage_out, dim3((words + 63) / 64), dim3(64), 0, E.stream, reinterpret_cast<const uint4*>(E.by),
-                       static_cast<uint4*>(my), words, dstatus, static_cast<uint32_t*>(ms));
+                       static_cast<uint4*>(my), words, E.bstatus, static_cast<uint32_t*>(ms));
     CK(hipStreamSynchronize(E.stream));
   } else {
-    CK(hipMemcpyAsync(E.bstatus_host, dstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, E.stream));
+    CK(hipMemcpyAsync(E.bstatus_host, E.bstatus, sizeof(uint32_t), hipMemcpyDeviceToHost, E.stream));
   }
   auto fetch = [&](size_t k) {   // piece k of y, if there is one
     const size_t at = k * kBatchPiece;

@@ -317,3 +317,39 @@ def test_prefill_captured_launch_records_kernels_only(eng):
         kind = C.c_int()
         assert hip.hipGraphNodeGetType(C.c_void_p(node), C.byref(kind)) == 0
         assert kind.value == 0, kind.value   # hipGraphNodeTypeKernel
+
+
+@pytest.mark.parametrize("tokens", [40, 130])
+def test_prefill_replayed_launch_keeps_its_status(eng, tokens):
+    """A captured fr_hip_batch_launch reports its own status at every replay, with
+    fr_hip_run_batch calls (by copy kernel at 40 tokens, in pieces at 130) and
+    eager work between the replays: a failing chunk's replay after a good
+    run_batch still fails, a good one after a failing run_batch still passes."""
+    import ctypes as C
+
+    import torch
+    hidden, lib = 4096, fa.lib()
+    load(eng, hidden, (0, 7))
+    rng = np.random.default_rng(tokens)
+    experts, gates, x = chunk(rng, tokens, hidden)
+    bad = x.copy()
+    bad[3, 5] = np.inf
+    good = run_ok(eng, 0, experts, gates, x)
+    plans = [eng.batch_plan(0, experts, gates, v, fa.MODE_F32) for v in (x, bad)]
+    dev = torch.from_numpy(plans[0]).to("cuda")
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
+        assert lib.fr_hip_batch_launch(plans[0].ctypes.data, dev.data_ptr(), C.c_void_p(s.cuda_stream)) == fa.OK
+    for rep in range(4):
+        fails = rep % 2 == 0
+        print(f"replay {rep}", flush=True)
+        rc, _ = eng.run_batch(0, experts, gates, x if fails else bad)
+        assert rc == (fa.OK if fails else fa.NUMERIC)
+        dev.copy_(torch.from_numpy(plans[1 if fails else 0]))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        y, status = np.zeros_like(x), C.c_uint()
+        assert lib.fr_hip_batch_output(None, fa.fptr(y), x.size, C.byref(status)) == fa.OK
+        assert (status.value != 0) == fails and np.array_equal(y, np.zeros_like(x) if fails else good), rep
