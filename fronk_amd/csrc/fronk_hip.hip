@@ -6884,8 +6884,8 @@ void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchSc
   else hipLaunchKernelGGL(prefill_gate_up<1>, g, b, 0, stream, dev_plan, S);
 }
 
-// `cleared`: the stream has zeroed the status word by then.
-int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream, bool cleared = false) {
+// What the launch refuses, and its scratch.
+int batch_ready(const BatchHeader& H) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
       H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
@@ -6893,7 +6893,12 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
     return FR_HIP_INVALID;
   const bool kt = H.gu == TQ4_KM && H.dn == TQ4_KT, nat = H.gu == TQ4_K && H.dn == TMXFP4;
   if (!kt && !nat) return FR_HIP_INVALID;
-  int rc = batch_scratch(H);
+  return batch_scratch(H);
+}
+
+// `cleared`: the stream has zeroed the status word by then.
+int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stream, bool cleared = false) {
+  const int rc = batch_ready(H);
   if (rc) return rc;
   BatchScratch S;
   S.h = E.bh;
@@ -6912,7 +6917,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
   const unsigned ncol = (H.hidden + kDownCols - 1) / kDownCols;
   hipLaunchKernelGGL(prefill_split, dim3(H.tokens), dim3(1024), 0, stream, dev_plan, S);
   const unsigned down_q8 = H.shtiles * ((H.hidden + down_rows_cols<TQ8_0>() - 1) / down_rows_cols<TQ8_0>());
-  if (kt) {
+  if (H.gu == TQ4_KM) {
     launch_gate_up(dev_plan, H, S, stream);
     if (H.shtiles)
       hipLaunchKernelGGL(prefill_gate_up_shared, dim3(H.shtiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
@@ -7414,10 +7419,7 @@ int fr_hip_batch_output(void* stream, float* y, size_t count, unsigned* status) 
   return batch_output(stream ? static_cast<hipStream_t>(stream) : E.stream, y, count, status);
 }
 
-int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
-  if (!g_open) return FR_HIP_STATE;
-  if (!req || !y) return FR_HIP_INVALID;
-  CK(hipSetDevice(E.device));
+static int run_batch(const fr_hip_batch* req, float* y) {
   if (req->tokens > (unsigned)kMaxBatchTokens) return FR_HIP_INVALID;
   const size_t need = (batch_capacity(req->tokens, req->hidden) + 15) & ~size_t(15);   // copied in 16-byte words
   if (need > E.bplan_cap) {
@@ -7442,6 +7444,8 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
     CK(hipHostMalloc(reinterpret_cast<void**>(&E.by_host), bytes, hipHostMallocMapped));
     E.by_host_bytes = bytes;
   }
+  rc = batch_ready(H);   // before anything is on its way
+  if (rc) return rc;
   // The plan with x goes up, y and the status come back through pinned memory of
   // the engine; y goes to the caller once the status is known. The status is
   // the engine's word, as in every batch launch, and is zeroed on the way up.
@@ -7500,10 +7504,7 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
   float ms = 0.f;
   if (hipEventElapsedTime(&ms, E.ev0, E.ev1) == hipSuccess) E.sample.last_kernel_ns = ms * 1e6;
   ++E.sample.runs;
-  if (status) {
-    CK(hipStreamSynchronize(E.stream));
-    return FR_HIP_NUMERIC;   // y is written only on success: untouched on failure
-  }
+  if (status) return FR_HIP_NUMERIC;   // y is written only on success: untouched on failure
   if (staged) {
     memcpy(y, E.by_host, bytes);
     return FR_HIP_OK;
@@ -7516,6 +7517,17 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
            bytes - at < kBatchPiece ? bytes - at : kBatchPiece);
   }
   return FR_HIP_OK;
+}
+
+int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
+  if (!g_open) return FR_HIP_STATE;
+  if (!req || !y) return FR_HIP_INVALID;
+  CK(hipSetDevice(E.device));
+  const int rc = run_batch(req, y);
+  // The next call writes the pinned plan and y at once: no copy of a call that
+  // fails half-way is left on its way.
+  if (rc) (void)hipStreamSynchronize(E.stream);
+  return rc;
 }
 
 int fr_hip_timing(unsigned launches) {
