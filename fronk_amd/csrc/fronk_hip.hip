@@ -4029,8 +4029,8 @@ struct BatchHeader {
   uint32_t nblk, layer, tiles_off, slots_off;
   uint32_t tokslot_off, x_off, total, experts;
   uint32_t nshared, shtiles, gu, dn;         // tokens with the shared expert, its tiles; routed formats
-  uint32_t gtiles_off, ngtiles;              // prefill_gate_up's tiles of the routed experts
-  uint32_t gslices, pad;                     // its slices per workgroup; 0: prefill_gate_up_few
+  uint32_t gtiles_off, ngtiles;              // prefill_gate_up's tiles of the routed experts (none: no launch reads them)
+  uint32_t gslices, pad;                     // its slices per workgroup; 0: prefill_gate_up_few or native units
   uint64_t slice_bytes, proj, shared_proj;
   uint64_t base[kBlocks];                // owned slices in ascending block order: the layer's base
 };
@@ -6669,7 +6669,7 @@ size_t batch_capacity(uint32_t tokens, uint32_t hidden) {
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 // How prefill_gate_up cuts the routed work: slices per workgroup (NB) and
-// 16-token tiles per workgroup (at most kGateUpTiles), or NB = 0 for
+// 16-token tiles per workgroup (at most kGateUpTiles), or NB = 0 and no tiles for
 // prefill_gate_up_few. Four slices per workgroup beat two and one (512 tokens,
 // 20 slices: 363, 430, 591 us; 4096 tokens: 1198, 1469, 2225) unless its last
 // wavefronts have no slice left, and larger tiles form each weight for more
@@ -6682,7 +6682,7 @@ GateUpCut gate_up_cut(const std::vector<uint32_t>& count, uint32_t nblk) {
   uint32_t n[kGateUpTiles + 1] = {};   // workgroup tiles at a cap
   for (uint32_t c : count)
     for (uint32_t cap = 1; cap <= (uint32_t)kGateUpTiles; ++cap) n[cap] += (c + kTileTokens * cap - 1) / (kTileTokens * cap);
-  GateUpCut best = {0, 1, n[1]};
+  GateUpCut best = {0, 0, 0};
   float least = 0.f;
   const struct { uint32_t nb; float cost; } kinds[] = {{4, 1.f}, {2, 1.2f}, {1, 1.65f}};
   for (const auto& k : kinds) {
@@ -6748,7 +6748,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used, b
     experts += count[id] ? 1u : 0u;
   }
   const uint32_t shtiles = (nshared + kTileTokens - 1) / kTileTokens;
-  const GateUpCut cut = gate_up_cut(count, H->nblk);
+  const GateUpCut cut = l0->gu == TQ4_KM ? gate_up_cut(count, H->nblk) : GateUpCut{0, 0, 0};
   H->hidden = hidden;
   H->tokens = T;
   H->nslots = nslots + nshared;
@@ -6889,9 +6889,10 @@ int batch_ready(const BatchHeader& H) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
       H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
-      !H.ngtiles || H.ngtiles > H.ntiles || (H.gslices != 0 && H.gslices != 1 && H.gslices != 2 && H.gslices != 4))
+      H.ngtiles > H.ntiles || !H.ngtiles != !H.gslices ||
+      (H.gslices != 0 && H.gslices != 1 && H.gslices != 2 && H.gslices != 4))
     return FR_HIP_INVALID;
-  const bool kt = H.gu == TQ4_KM && H.dn == TQ4_KT, nat = H.gu == TQ4_K && H.dn == TMXFP4;
+  const bool kt = H.gu == TQ4_KM && H.dn == TQ4_KT, nat = H.gu == TQ4_K && H.dn == TMXFP4 && !H.gslices;
   if (!kt && !nat) return FR_HIP_INVALID;
   return batch_scratch(H);
 }

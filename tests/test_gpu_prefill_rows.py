@@ -293,3 +293,16 @@ def test_prefill_rows_mx_exponent_edges(eng):
         for v, g in zip(views, goods):
             v[:] = g
         refresh()
+
+
+def test_native_plans_carry_no_unread_tiles(eng):
+    """Plans whose launch reads no prefill_gate_up tiles hold none: native units,
+    and Q4_K-T chunks on prefill_gate_up_few."""
+    hidden, blocks = 2560, (0, 7)
+    rng = np.random.default_rng(3)
+    for fmt in (fa.FMT_NATIVE, fa.FMT_Q4KT):
+        load(eng, hidden, blocks, fmt)
+        experts, gates, x = chunk(rng, 20, hidden, rng.choice(512, 40, replace=False))
+        plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+        assert not plan[68:76].view(np.uint32).any()   # BatchHeader.ngtiles, gslices
+        assert eng.run_batch(0, experts, gates, x)[0] == fa.OK
