@@ -7432,6 +7432,7 @@ static int run_batch(const fr_hip_batch* req, float* y) {
     CK(hipMalloc(&E.bplan_dev, need));
     CK(hipHostMalloc(reinterpret_cast<void**>(&E.bplan_host), need, hipHostMallocMapped));
     E.bplan_cap = need;
+    ++E.sample.hot_allocations;
   }
   size_t used = 0;
   int rc = build_batch(req, E.bplan_host, E.bplan_cap, &used, false);
@@ -7444,6 +7445,7 @@ static int run_batch(const fr_hip_batch* req, float* y) {
     E.by_host_bytes = 0;
     CK(hipHostMalloc(reinterpret_cast<void**>(&E.by_host), bytes, hipHostMallocMapped));
     E.by_host_bytes = bytes;
+    ++E.sample.hot_allocations;
   }
   rc = batch_ready(H);   // before anything is on its way
   if (rc) return rc;

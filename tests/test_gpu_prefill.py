@@ -353,3 +353,26 @@ def test_prefill_replayed_launch_keeps_its_status(eng, tokens):
         y, status = np.zeros_like(x), C.c_uint()
         assert lib.fr_hip_batch_output(None, fa.fptr(y), x.size, C.byref(status)) == fa.OK
         assert (status.value != 0) == fails and np.array_equal(y, np.zeros_like(x) if fails else good), rep
+
+
+def test_prefill_buffers_count_as_hot_allocations(eng):
+    """Every buffer that a chunk grows is in the sample's hot_allocations: the
+    scratch (four buffers) by the launch, run_batch's plan and y by its first
+    call at a size, none by the second."""
+    import torch
+    hidden, lib = 2560, fa.lib()
+    load(eng, hidden, ())
+    assert eng.close() == fa.OK   # the next engine has no scratch
+    fa.Engine(0)
+    load(eng, hidden, (0,))
+    experts, gates, x = chunk(np.random.default_rng(1), 20, hidden)
+    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+    dev = torch.from_numpy(plan).to("cuda")
+    torch.cuda.synchronize()
+    assert eng.sample().hot_allocations == 0
+    assert lib.fr_hip_batch_launch(plan.ctypes.data, dev.data_ptr(), None) == fa.OK
+    assert lib.fr_hip_batch_output(None, None, 0, None) == fa.OK
+    assert eng.sample().hot_allocations == 4
+    for _ in range(2):
+        run_ok(eng, 0, experts, gates, x)
+        assert eng.sample().hot_allocations == 6
