@@ -4030,7 +4030,7 @@ struct BatchHeader {
   uint32_t tokslot_off, x_off, total, experts;
   uint32_t nshared, shtiles, gu, dn;         // tokens with the shared expert, its tiles; routed formats
   uint32_t gtiles_off, ngtiles;              // prefill_gate_up's tiles of the routed experts (none: no launch reads them)
-  uint32_t gslices, pad;                     // its slices per workgroup; 0: prefill_gate_up_few or native units
+  uint32_t gslices, gdown;                   // its slices per workgroup; 0: prefill_gate_up_few or native units. Then prefill_down?
   uint64_t slice_bytes, proj, shared_proj;
   uint64_t base[kBlocks];                // owned slices in ascending block order: the layer's base
 };
@@ -4203,8 +4203,8 @@ struct GateUpLds {
 //
 // What bounds it: with many tokens per expert the matrix cores, if the
 // operands reach them: an x' operand is read from LDS once per NB products of
-// 16 cycles (at NB = 1 LDS alone would take twice the products' time), a
-// weight is formed once per MT tiles, and a workgroup's NB slices share one
+// 16 cycles (at NB = 1 LDS alone would take twice the products' time: never
+// the best of the three), a weight is formed once per MT tiles, and a workgroup's NB slices share one
 // copy of the x' that each CU reads from L2 (16 KB per token). With few, the
 // weights' way from memory.
 // x' goes from memory to LDS without passing registers, half a super-block
@@ -4453,7 +4453,7 @@ __global__ __launch_bounds__(kGateUpThreads, 2) void prefill_gate_up(const uint8
 }
 
 
-// The same for chunks too small to give every CU its workgroups above: one
+// The same where prefill_cut finds it faster, as for few slices: one
 // slice and 16 tokens per workgroup of eight wavefronts. Wavefront w takes row-block w%4 (gate rows of
 // neurons 8rb..8rb+7, then their up rows) and part w/4 (sub-blocks 0-3 or 4-7
 // of every super-block), so that a wavefront's serial run over the row is half
@@ -4924,10 +4924,10 @@ __global__ __launch_bounds__(kDownThreads, 4) void prefill_down(const uint8_t* _
   if (bad) flag(S.status, bad);
 }
 
-// The down of chunks that prefill_gate_up_few takes (16-token tiles): each
-// wavefront forms B for itself and needs no barrier, which is the better
-// bargain for few slices (64 tokens, one slice, hidden 4096: the whole launch
-// 54 us, 66 us with prefill_down; 200 tokens, seven slices: 202 and 207 us).
+// The same where prefill_cut finds it faster (16-token tiles): each wavefront
+// forms B for itself and needs no barrier, which is the better bargain for few
+// slices and small tiles (hidden 4096: 64 tokens on one slice 23 us, 36 with
+// prefill_down; 250 on seven 81 us against 100).
 // Workgroup (tile, 512 outputs), four wavefronts: wavefront w takes the 128
 // outputs 256 sb + 128 hb .. +127 (sb = 2 blockIdx.y + w/2, hb = w%2), eight
 // 16-output tiles in one pass over all owned slices (B, the slice's header
@@ -6668,31 +6668,69 @@ size_t batch_capacity(uint32_t tokens, uint32_t hidden) {
 
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
-// How prefill_gate_up cuts the routed work: slices per workgroup (NB) and
-// 16-token tiles per workgroup (at most kGateUpTiles), or NB = 0 and no tiles for
-// prefill_gate_up_few. Four slices per workgroup beat two and one (512 tokens,
-// 20 slices: 363, 430, 591 us; 4096 tokens: 1198, 1469, 2225) unless its last
-// wavefronts have no slice left, and larger tiles form each weight for more
-// tokens; both need about four workgroups per CU (two resident), or the last
-// ones run alone.
-struct GateUpCut {
-  uint32_t nb, cap, tiles;
+// A launch's time in times of one workgroup, `slots` of n running at once: a
+// partly filled last turn costs what its workgroups share a CU with.
+float launch_turns(float n, float slots) {
+  const float q = n / slots;
+  return q <= 0.5f ? 0.65f : q <= 1.f ? 1.f : q <= 1.5f ? 1.4f : q <= 2.f ? 1.9f : q;
+}
+
+// Which kernels take the routed work of a Q4_K-T chunk (`pairs` (token, expert)s
+// in `ntiles` 16-token tiles).
+//
+// The gate/up: prefill_gate_up with NB = `nb` slices and up to `cap` 16-token
+// tiles per workgroup (`tiles` of them), or prefill_gate_up_few (nb = 0), by the
+// time of their workgroups: two of each kernel run on a CU, one turn's time per
+// super-block of the row is 1.4 us for _few, 4.3, 6.3, 9.6 and 11.4 us with
+// four slices and 1 to 4 tiles, 2.55, 3.75, 5.7 and 7.1 with two. A last
+// workgroup's wavefronts without a slice, a poorly filled turn and the tiles that
+// an XCD has more than its neighbours count, larger tiles form each weight for
+// more tokens and are taken as long as they leave four workgroups per CU. Over
+// 594 chunks (24 to 4096 tokens; uniform, skewed and 40-expert routing; 1 to 20
+// slices; hidden 2560 and 4096) the gate/up it takes is 0.4 % slower than the
+// best of the three on average, and 4 % slower than _few at most. At hidden 4096,
+// 100 uniform tokens on 4 slices: 64 us with four slices per workgroup, 74 with
+// two, 80 _few; 160 on 3: 64, 73, 67; 2200 on 4: 227, 176, 294; 2200 on 1: _few
+// 84 us, 136 with two.
+//
+// The down: prefill_down where its workgroups' tokens times the slices make up
+// for its barriers and its B of four slices at a time, prefill_down_few
+// otherwise. The line lies at 6 tokens for 20 slices, 12 for 10, 24 for 5 (hidden
+// 4096, uniform tokens: 100 on 20 slices, 2.3 per workgroup, 180 us against 175
+// _few; 400, 7.8, 203 against 245; 400 on 10, 7.8, 124 against 111; 700, 13.7, 140
+// against 150; 700 on 5, 13.7, 101 against 86; 2200, 43, 216 against 254); the
+// way it takes is 0.6 % slower than the better one on average.
+struct PrefillCut {
+  uint32_t nb, cap, tiles, down;
 };
-GateUpCut gate_up_cut(const std::vector<uint32_t>& count, uint32_t nblk) {
-  uint32_t n[kGateUpTiles + 1] = {};   // workgroup tiles at a cap
-  for (uint32_t c : count)
-    for (uint32_t cap = 1; cap <= (uint32_t)kGateUpTiles; ++cap) n[cap] += (c + kTileTokens * cap - 1) / (kTileTokens * cap);
-  GateUpCut best = {0, 0, 0};
-  float least = 0.f;
-  const struct { uint32_t nb; float cost; } kinds[] = {{4, 1.f}, {2, 1.2f}, {1, 1.65f}};
-  for (const auto& k : kinds) {
-    const uint32_t groups = (nblk + k.nb - 1) / k.nb;
-    const float cost = k.cost * (float)(groups * k.nb);
-    if ((best.nb && cost >= least) || n[1] * groups < 4 * E.cus) continue;
-    uint32_t cap = kGateUpTiles;
-    while (cap > 1 && n[cap] * groups < 4 * E.cus) --cap;
-    best = {k.nb, cap, n[cap]};
-    least = cost;
+PrefillCut prefill_cut(const std::vector<uint32_t>& count, uint32_t pairs, uint32_t ntiles, uint32_t nblk) {
+  static const float turn[2][kGateUpTiles] = {{4.3f, 6.3f, 9.6f, 11.4f}, {2.55f, 3.75f, 5.7f, 7.1f}};
+  const float slots = 2.f * (float)E.cus;
+  PrefillCut best = {0, 0, 0, 0};
+  float least = 1.4f * launch_turns((float)(ntiles * nblk), slots);
+  for (uint32_t k = 0; k < 2; ++k) {
+    const uint32_t nb = k ? 2 : 4, groups = (nblk + nb - 1) / nb;
+    uint32_t cap = kGateUpTiles + 1, tiles = 0;
+    uint32_t len[kGateUpTiles + 1];   // workgroup tiles of 1..cap 16-token tiles
+    do {
+      --cap;
+      tiles = 0;
+      memset(len, 0, sizeof(len));
+      for (uint32_t c : count) {
+        const uint32_t nt = (c + kTileTokens - 1) / kTileTokens, n = (nt + cap - 1) / cap;
+        if (!n) continue;
+        tiles += n;
+        len[nt / n] += n - nt % n;
+        if (nt % n) len[nt / n + 1] += nt % n;
+      }
+    } while (cap > 1 && tiles * groups < 4 * E.cus);
+    float mean = 0.f;
+    for (uint32_t m = 1; m <= cap; ++m) mean += (float)len[m] / (float)tiles * turn[k][m - 1];
+    const float time = mean * launch_turns((float)((tiles + 7) / 8 * 8 * groups), slots);
+    if (time < least) {
+      least = time;
+      best = {nb, cap, tiles, nblk * pairs >= 120 * tiles ? 1u : 0u};
+    }
   }
   return best;
 }
@@ -6748,7 +6786,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used, b
     experts += count[id] ? 1u : 0u;
   }
   const uint32_t shtiles = (nshared + kTileTokens - 1) / kTileTokens;
-  const GateUpCut cut = l0->gu == TQ4_KM ? gate_up_cut(count, H->nblk) : GateUpCut{0, 0, 0};
+  const PrefillCut cut = l0->gu == TQ4_KM ? prefill_cut(count, nslots, ntiles, H->nblk) : PrefillCut{0, 0, 0, 0};
   H->hidden = hidden;
   H->tokens = T;
   H->nslots = nslots + nshared;
@@ -6766,6 +6804,7 @@ int build_batch(const fr_hip_batch* r, uint8_t* out, size_t cap, size_t* used, b
   H->gtiles_off = (uint32_t)align256(H->tiles_off + (size_t)(ntiles + shtiles) * sizeof(BatchTile));
   H->ngtiles = cut.tiles;
   H->gslices = cut.nb;
+  H->gdown = cut.down;
   H->slots_off = (uint32_t)align256(H->gtiles_off + (size_t)cut.tiles * sizeof(BatchTile));
   H->tokslot_off = (uint32_t)align256(H->slots_off + (size_t)H->nslots * sizeof(BatchSlot));
   H->x_off = (uint32_t)align256(H->tokslot_off + (size_t)T * 11 * sizeof(uint32_t));
@@ -6872,7 +6911,7 @@ int batch_scratch(const BatchHeader& H) {
 // memset node in a graph has given wrong results on replays after the first.
 __global__ void clear_word(uint32_t* w) { *w = 0; }
 
-// Routed gate/up of all-Q4_K units (gate_up_cut).
+// Routed gate/up of all-Q4_K units (prefill_cut).
 void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchScratch& S, hipStream_t stream) {
   if (!H.gslices) {
     hipLaunchKernelGGL(prefill_gate_up_few, dim3(H.ntiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
@@ -6880,8 +6919,7 @@ void launch_gate_up(const uint8_t* dev_plan, const BatchHeader& H, const BatchSc
   }
   const dim3 g((H.ngtiles + 7) / 8 * 8 * ((H.nblk + H.gslices - 1) / H.gslices)), b(kGateUpThreads);
   if (H.gslices == 4) hipLaunchKernelGGL(prefill_gate_up<4>, g, b, 0, stream, dev_plan, S);
-  else if (H.gslices == 2) hipLaunchKernelGGL(prefill_gate_up<2>, g, b, 0, stream, dev_plan, S);
-  else hipLaunchKernelGGL(prefill_gate_up<1>, g, b, 0, stream, dev_plan, S);
+  else hipLaunchKernelGGL(prefill_gate_up<2>, g, b, 0, stream, dev_plan, S);
 }
 
 // What the launch refuses, and its scratch.
@@ -6889,8 +6927,8 @@ int batch_ready(const BatchHeader& H) {
   if (!H.tokens || H.tokens > (unsigned)kMaxBatchTokens || !H.ntiles || !H.nblk || H.nblk > (unsigned)kBlocks ||
       !H.hidden || H.hidden % 256 || H.hidden > (unsigned)kMaxHidden || H.nshared > H.tokens ||
       H.nslots != 10 * H.tokens + H.nshared || H.shtiles != (H.nshared + kTileTokens - 1) / kTileTokens ||
-      H.ngtiles > H.ntiles || !H.ngtiles != !H.gslices ||
-      (H.gslices != 0 && H.gslices != 1 && H.gslices != 2 && H.gslices != 4))
+      H.ngtiles > H.ntiles || !H.ngtiles != !H.gslices || (H.gslices != 0 && H.gslices != 2 && H.gslices != 4) ||
+      H.gdown > (H.gslices ? 1u : 0u))
     return FR_HIP_INVALID;
   const bool kt = H.gu == TQ4_KM && H.dn == TQ4_KT, nat = H.gu == TQ4_K && H.dn == TMXFP4 && !H.gslices;
   if (!kt && !nat) return FR_HIP_INVALID;
@@ -6922,7 +6960,7 @@ int batch_launch(const uint8_t* dev_plan, const BatchHeader& H, hipStream_t stre
     launch_gate_up(dev_plan, H, S, stream);
     if (H.shtiles)
       hipLaunchKernelGGL(prefill_gate_up_shared, dim3(H.shtiles * H.nblk), dim3(kBatchThreads), 0, stream, dev_plan, S);
-    if (H.gslices)
+    if (H.gdown)
       hipLaunchKernelGGL(prefill_down, dim3((H.ngtiles + 7) / 8 * 8 * (H.hidden / 256)), dim3(kDownThreads), 0, stream,
                          dev_plan, S);
     else

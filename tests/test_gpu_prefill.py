@@ -240,23 +240,27 @@ def test_prefill_down_operand_parts_agree(eng):
             assert rc == 0 and err[0] <= 2e-6, (seed, t, err)
 
 
-@pytest.mark.parametrize("hidden,nblk,tokens,pool,slices", [
-    (2560, 20, 200, 300, 4),    # tiles of one to four 16-token tiles, all with partial ends
-    (2304, 7, 700, 512, 4),     # nine super-blocks; the last workgroup's fourth wavefront has no slice
-    (2304, 6, 160, 512, 2),
-    (256, 1, 2600, 512, 1),     # one super-block
-    (4096, 3, 24, 30, 0),       # too few workgroups: prefill_gate_up_few
+@pytest.mark.parametrize("hidden,nblk,tokens,pool,slices,down", [
+    (2560, 20, 200, 300, 4, 1),    # tiles of one to four 16-token tiles, all with partial ends
+    (2304, 7, 700, 512, 4, 0),     # nine super-blocks; the last workgroup's fourth wavefront has no slice
+    (2304, 10, 900, 512, 2, 1),
+    (2304, 7, 1600, 512, 4, 1),
+    (2304, 6, 160, 512, 2, 0),
+    (2560, 18, 130, 512, 4, 0),    # two wavefronts of the last workgroup without a slice
+    (256, 20, 600, 100, 4, 1),     # one super-block
+    (256, 1, 2600, 512, 0, 0),     # one super-block and slice
+    (4096, 3, 24, 30, 0, 0),       # few workgroups
 ])
-def test_prefill_gate_up_cuts(eng, hidden, nblk, tokens, pool, slices):
-    """Each way the routed gate/up is cut into workgroups, at odd sizes: rows
-    against the oracle, and a repeat bit for bit."""
+def test_prefill_gate_up_cuts(eng, hidden, nblk, tokens, pool, slices, down):
+    """Each way the routed gate/up is cut into workgroups, with either down, at odd
+    sizes: rows against the oracle, and a repeat bit for bit."""
     blocks = tuple(range(20 - nblk, 20))
     lay = oracle.layout(hidden, fa.FMT_Q4KT)
     load(eng, hidden, blocks)
     rng = np.random.default_rng(hidden + tokens)
     experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
     plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
-    assert plan[72:76].view(np.uint32)[0] == slices   # BatchHeader.gslices
+    assert plan[72:80].view(np.uint32).tolist() == [slices, down]   # BatchHeader.gslices, gdown
     y = run_ok(eng, 0, experts, gates, x)
     assert np.array_equal(y, run_ok(eng, 0, experts, gates, x))
     rows = rng.choice(tokens, 7, replace=False)
