@@ -4627,7 +4627,11 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
 //     MTP (MT up to a power of two) token tiles a round takes RS = 4/MTP
 //     slices, wavefront w forms (slice w/MTP, token tile w%MTP);
 //   the min terms' A[g][n] = m_ng, B = dmin_n h'_nt in two parts, by the same
-//     wavefront, eight of sixteen rows in use.
+//     wavefront, eight of sixteen rows in use (as fp32 products they cost 11 % of
+//     the kernel at 4096 tokens and leave the same error against 64 bits, 1.1e-7).
+// A neuron's |dmin| below 2^-8 enters B 1024 times as large and its m A 1024
+// times as small (exact, and normal), so that the smallest scale's product with
+// the largest h' is 2^-2 and keeps its 22 bits above f16's floor of 2^-24.
 // The products add straight into the accumulators over the slices. The rounds
 // are pipelined behind one barrier each: while round i's products run, round
 // i+1's B is formed and the scales of round i+2 are unpacked.
@@ -4642,12 +4646,13 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
 // tokens). Measured, 20 slices at hidden 4096, against prefill_down_few:
 // 512 tokens 200 (215) us, 4096 tokens 730 (1100) us.
 constexpr float kDownDirect = 4.f;
+constexpr uint32_t kDownSmall = 0x1c00;      // bits of the f16 2^-8
 constexpr int kDownThreads = 256, kDownWaves = kDownThreads / 64;
 struct DownLds {
   // [round mod 3][slice of the round]
   _Float16 sc[3][4][8][kNeurons];            // 6-bit scale of (sub-block, neuron)
-  _Float16 mn[3][4][8][kNeurons];            // 6-bit min
-  float d[3][4][kNeurons], dm[3][4][kNeurons];
+  _Float16 mn[3][4][8][kNeurons];            // 6-bit min, over 1024 for a small dmin
+  float d[3][4][kNeurons], dm[3][4][kNeurons];   // d; dmin, times 1024 where it is small
   uint4 b[2][kDownWaves][2][64];             // [round mod 2][slice, token tile][part][lane]: B
   float corr[kDownWaves][8][kTileTokens];    // each wavefront's min terms [sub-block][token]
   uint32_t deferred;                         // slices with a large d or dmin (bit R)
@@ -4719,16 +4724,19 @@ __device__ __forceinline__ void down_tile(const BatchHeader& H, const BatchScrat
   // Scales of sub-blocks g0..g0+n-1 of the thread's neuron into table (buf, r).
   auto unpack = [&](const u32x4& hd, unsigned buf, unsigned r, unsigned g0, unsigned n) {
     hflag |= half_bad_bits(hd[0]);
+    const bool smallm = (hd[0] >> 16 & 0x7fffu) < kDownSmall;
+    const f16x2 f = {(_Float16)1.f, smallm ? (_Float16)0x1p-10f : (_Float16)1.f};
 #pragma unroll
     for (unsigned i = 0; i < n; ++i) {
       uint32_t sc, mi;
       q4k_scale_min(hd[1], hd[2], hd[3], g0 + i, sc, mi);
-      L.sc[buf][r][g0 + i][hn] = (_Float16)(unsigned short)sc;
-      L.mn[buf][r][g0 + i][hn] = (_Float16)(unsigned short)mi;
+      const f16x2 v = f * (f16x2){(_Float16)(unsigned short)sc, (_Float16)(unsigned short)mi};
+      L.sc[buf][r][g0 + i][hn] = v[0];
+      L.mn[buf][r][g0 + i][hn] = v[1];
     }
     if (g0 == 0) {
       L.d[buf][r][hn] = half_to_float(hd[0] & 0xffffu);
-      L.dm[buf][r][hn] = half_to_float(hd[0] >> 16);
+      L.dm[buf][r][hn] = half_to_float(hd[0] >> 16) * (smallm ? 1024.f : 1.f);
     }
   };
   // 256/RS threads per slice, RS sub-blocks each.

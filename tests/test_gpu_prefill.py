@@ -380,3 +380,50 @@ def test_prefill_buffers_count_as_hot_allocations(eng):
     for _ in range(2):
         run_ok(eng, 0, experts, gates, x)
         assert eng.sample().hot_allocations == 6
+
+
+@pytest.mark.parametrize("nblk,tokens,pool,slices", [(20, 320, 300, 4), (2, 24, 30, 0)])
+@pytest.mark.parametrize("what", ["min"])
+def test_prefill_small_down_scales(eng, what, nblk, tokens, pool, slices):
+    """The down of an expert whose fp16 scales are the smallest there are (d and
+    dmin 2^-24 to 3 * 2^-24, or d zero and y the min terms alone), on the tokens
+    for which it is the only expert with a gate. The main sum has operands of 22
+    bits and fp32 sums, the min terms are fp32: at most 2e-6 of a row, as with
+    larger scales (operands with f16's absolute floor of 2^-25 would be off by
+    2^-13 and more of their largest)."""
+    hidden, blocks = 2560, tuple(range(20 - nblk, 20))
+    lay = oracle.layout(hidden, fa.FMT_Q4KT)
+    load(eng, hidden, blocks)
+    rng = np.random.default_rng(31 + nblk)
+    experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
+    count = np.bincount(experts.ravel(), minlength=512)
+    chosen = [int(np.argmax(count)), int(np.flatnonzero(count == count[count > 0].min())[0])]   # a hot and a cold one
+    rows = []
+    for e in chosen:
+        for t in np.flatnonzero((experts == e).any(axis=1))[:10]:
+            if int(t) not in rows:
+                gates[t, :10] = np.where(experts[t] == e, gates[t, :10], 0)
+                rows.append(int(t))
+    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+    assert plan[72:80].view(np.uint32).tolist() == [slices, 1 if slices else 0]   # BatchHeader.gslices, gdown
+    units = host_units(lay, blocks, 0, chosen)
+    try:
+        for b in blocks:
+            for e in chosen:
+                view = slice_view(units[b], lay, 0, e)
+                head = view[2 * lay.proj:2 * lay.proj + 32 * lay.down_row].reshape(-1, 144)   # a super-block each
+                d = rng.integers(1, 4, (len(head), 2)).astype(np.uint16)                       # fp16 subnormals
+                if what == "min":
+                    d[:, 0] = 0
+                head[:, :4] = d.view(np.uint8).reshape(-1, 4)
+                assert eng.refresh(b, units[b], 0, e) == fa.OK
+        y = run_ok(eng, 0, experts, gates, x)
+        for i in range(0, len(rows), 8):
+            part = rows[i:i + 8]
+            rc, ref = oracle.ref_run(units, fa.FMT_Q4KT, False, oracle_request(0, experts[part], gates[part], x[part]))
+            assert rc == 0
+            for j, t in enumerate(part):
+                rc, err = oracle.compare(ref[j], y[t])
+                assert rc == 0 and err[0] <= 2e-6, (what, t, err)
+    finally:
+        load(eng, hidden, ())
