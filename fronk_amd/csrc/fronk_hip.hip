@@ -2112,6 +2112,11 @@ __device__ __forceinline__ uint32_t scaled_u16(uint32_t p, uint32_t sc2) {
   const f16x2 f = __builtin_bit_cast(f16x2, m) - (f16x2){(_Float16)1024.f, (_Float16)1024.f};
   return __builtin_bit_cast(uint32_t, f);
 }
+// The same times a power of two, f = {2^-k, 2^-k}, b = {-2^(10-k), -2^(10-k)}.
+__device__ __forceinline__ uint32_t scaled_u16(uint32_t p, uint32_t sc2, f16x2 f, f16x2 b) {
+  const u16x2 m = __builtin_bit_cast(u16x2, p) * __builtin_bit_cast(u16x2, sc2) + (u16x2){0x6400, 0x6400};
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2, m), f, b));
+}
 // Bytes 2H, 2H+1 of v (each below 16) times sch (two f16 copies of a 6-bit
 // scale) as two exact normal f16 values sc*q, in two instructions: a byte
 // below 16 read as FP8 E4M3 is q * 2^-9 exactly, v_cvt_scalef32_pk_f16_fp8
@@ -4629,8 +4634,8 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
 //   the min terms' A[g][n] = m_ng, B = dmin_n h'_nt in two parts, by the same
 //     wavefront, eight of sixteen rows in use (as fp32 products they cost 11 % of
 //     the kernel at 4096 tokens and leave the same error against 64 bits, 1.1e-7).
-// A neuron's |dmin| below 2^-8 enters B 1024 times as large and its m A 1024
-// times as small (exact, and normal), so that the smallest scale's product with
+// A neuron's |d| or |dmin| below 2^-8 enters B 1024 times as large and its sc q or
+// m A 1024 times as small (exact, and normal), so that the smallest scale's product with
 // the largest h' is 2^-2 and keeps its 22 bits above f16's floor of 2^-24.
 // The products add straight into the accumulators over the slices. The rounds
 // are pipelined behind one barrier each: while round i's products run, round
@@ -4650,9 +4655,9 @@ constexpr uint32_t kDownSmall = 0x1c00;      // bits of the f16 2^-8
 constexpr int kDownThreads = 256, kDownWaves = kDownThreads / 64;
 struct DownLds {
   // [round mod 3][slice of the round]
-  _Float16 sc[3][4][8][kNeurons];            // 6-bit scale of (sub-block, neuron)
+  _Float16 sc[3][4][8][kNeurons];            // 6-bit scale of (sub-block, neuron), over 1024 for a small d
   _Float16 mn[3][4][8][kNeurons];            // 6-bit min, over 1024 for a small dmin
-  float d[3][4][kNeurons], dm[3][4][kNeurons];   // d; dmin, times 1024 where it is small
+  float d[3][4][kNeurons], dm[3][4][kNeurons];   // d and dmin, times 1024 where they are small
   uint4 b[2][kDownWaves][2][64];             // [round mod 2][slice, token tile][part][lane]: B
   float corr[kDownWaves][8][kTileTokens];    // each wavefront's min terms [sub-block][token]
   uint32_t deferred;                         // slices with a large d or dmin (bit R)
@@ -4724,8 +4729,8 @@ __device__ __forceinline__ void down_tile(const BatchHeader& H, const BatchScrat
   // Scales of sub-blocks g0..g0+n-1 of the thread's neuron into table (buf, r).
   auto unpack = [&](const u32x4& hd, unsigned buf, unsigned r, unsigned g0, unsigned n) {
     hflag |= half_bad_bits(hd[0]);
-    const bool smallm = (hd[0] >> 16 & 0x7fffu) < kDownSmall;
-    const f16x2 f = {(_Float16)1.f, smallm ? (_Float16)0x1p-10f : (_Float16)1.f};
+    const bool small = (hd[0] & 0x7fffu) < kDownSmall, smallm = (hd[0] >> 16 & 0x7fffu) < kDownSmall;
+    const f16x2 f = {small ? (_Float16)0x1p-10f : (_Float16)1.f, smallm ? (_Float16)0x1p-10f : (_Float16)1.f};
 #pragma unroll
     for (unsigned i = 0; i < n; ++i) {
       uint32_t sc, mi;
@@ -4735,7 +4740,7 @@ __device__ __forceinline__ void down_tile(const BatchHeader& H, const BatchScrat
       L.mn[buf][r][g0 + i][hn] = v[1];
     }
     if (g0 == 0) {
-      L.d[buf][r][hn] = half_to_float(hd[0] & 0xffffu);
+      L.d[buf][r][hn] = half_to_float(hd[0] & 0xffffu) * (small ? 1024.f : 1.f);
       L.dm[buf][r][hn] = half_to_float(hd[0] >> 16) * (smallm ? 1024.f : 1.f);
     }
   };
@@ -4949,7 +4954,8 @@ __global__ __launch_bounds__(kDownThreads, 4) void prefill_down(const uint8_t* _
 // v_mfma_f32_16x16x32_f16 over the 32 neurons (lane group kq: neurons
 // 8kq..8kq+7):
 //   A[o][n] = sc_ng * q_on exactly in f16 (sc q < 1024), a packed 16-bit
-//     multiply-add and an f16 subtraction per two neurons (scaled_u16);
+//     multiply-add and an f16 fused multiply-add per two neurons (scaled_u16),
+//     over 1024 (and B times 1024) in a slice whose |d| are all below 2^-8;
 //   B[n][t] = d_n h'_nt in two f16 parts (22 significant bits), formed once
 //     per slice for the wavefront's eight tiles;
 // and the products add straight into the tiles' accumulators over the
@@ -4969,7 +4975,7 @@ struct DownFewLds {
   // [wave][slice parity][sub-block 4hb + j of the wavefront][neuron]
   uint16_t sc[kDownWaves][2][4][kNeurons];   // 6-bit scale
   float mm[kDownWaves][2][4][kNeurons];      // dmin * m
-  float d[kDownWaves][2][kNeurons];          // d
+  float d[kDownWaves][2][kNeurons];          // d, times 1024 in a slice of small d
 };
 
 __global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_t* __restrict__ plan, BatchScratch S) {
@@ -5033,8 +5039,9 @@ __global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_
       B.h = __builtin_amdgcn_raw_buffer_load_b128(rs, (int)vh, 0, 0);
     };
     // The slice's header table (parity par): lane l decodes neuron l%32 for
-    // sub-blocks j = l/32 and 2 + l/32. Returns whether the neuron's d takes
-    // the direct path.
+    // sub-blocks j = l/32 and 2 + l/32; fa and fb: scaled_u16's factors for it.
+    // Returns whether the neuron's d takes the direct path.
+    f16x2 fa, fb;
     auto table = [&](const u32x4& hd, unsigned par) {
       hflag |= half_bad_bits(hd[0]);
       const float dn = half_to_float(hd[0] & 0xffff), dmn = half_to_float(hd[0] >> 16);
@@ -5045,7 +5052,10 @@ __global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_
       L.sc[wave][par][2 + hgg][hn] = (uint16_t)sc1;
       L.mm[wave][par][hgg][hn] = dmn * (float)mi0;
       L.mm[wave][par][2 + hgg][hn] = dmn * (float)mi1;
-      if (hgg == 0) L.d[wave][par][hn] = dn;
+      const bool small = __ballot((hd[0] & 0x7fffu) >= kDownSmall) == 0;
+      fa = __builtin_bit_cast(f16x2, small ? 0x14001400u : 0x3c003c00u);   // 2^-10 or 1
+      fb = __builtin_bit_cast(f16x2, small ? 0xbc00bc00u : 0xe400e400u);   // -1 or -1024
+      if (hgg == 0) L.d[wave][par][hn] = small ? 1024.f * dn : dn;
       __builtin_amdgcn_wave_barrier();
       return fabsf(dn) < kDownDirect;
     };
@@ -5070,10 +5080,10 @@ __global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_
       constexpr int PH = decltype(ph)::value, MQ = decltype(mq)::value;
       const uint4 s4 = *reinterpret_cast<const uint4*>(&L.sc[wave][par][2 * PH + MQ / 2][8 * kq]);
       const u32x4& U = B.u[PH];
-      const u32x4 aw = {scaled_u16(quad_nibbles<MQ>(U[0], mask, shift), s4.x),
-                        scaled_u16(quad_nibbles<MQ>(U[1], mask, shift), s4.y),
-                        scaled_u16(quad_nibbles<MQ>(U[2], mask, shift), s4.z),
-                        scaled_u16(quad_nibbles<MQ>(U[3], mask, shift), s4.w)};
+      const u32x4 aw = {scaled_u16(quad_nibbles<MQ>(U[0], mask, shift), s4.x, fa, fb),
+                        scaled_u16(quad_nibbles<MQ>(U[1], mask, shift), s4.y, fa, fb),
+                        scaled_u16(quad_nibbles<MQ>(U[2], mask, shift), s4.z, fa, fb),
+                        scaled_u16(quad_nibbles<MQ>(U[3], mask, shift), s4.w, fa, fb)};
       return __builtin_bit_cast(f16x8, aw);
     };
     using I0 = std::integral_constant<int, 0>;

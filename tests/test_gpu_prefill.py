@@ -383,7 +383,7 @@ def test_prefill_buffers_count_as_hot_allocations(eng):
 
 
 @pytest.mark.parametrize("nblk,tokens,pool,slices", [(20, 320, 300, 4), (2, 24, 30, 0)])
-@pytest.mark.parametrize("what", ["min"])
+@pytest.mark.parametrize("what", ["min", "both"])
 def test_prefill_small_down_scales(eng, what, nblk, tokens, pool, slices):
     """The down of an expert whose fp16 scales are the smallest there are (d and
     dmin 2^-24 to 3 * 2^-24, or d zero and y the min terms alone), on the tokens
