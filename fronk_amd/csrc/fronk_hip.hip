@@ -7476,7 +7476,8 @@ int fr_hip_batch_output(void* stream, float* y, size_t count, unsigned* status) 
   return batch_output(stream ? static_cast<hipStream_t>(stream) : E.stream, y, count, status);
 }
 
-static int run_batch(const fr_hip_batch* req, float* y) {
+// `sent` is set once something is on its way on the engine's stream.
+static int run_batch(const fr_hip_batch* req, float* y, bool& sent) {
   if (req->tokens > (unsigned)kMaxBatchTokens) return FR_HIP_INVALID;
   const size_t need = (batch_capacity(req->tokens, req->hidden) + 15) & ~size_t(15);   // copied in 16-byte words
   if (need > E.bplan_cap) {
@@ -7514,6 +7515,7 @@ static int run_batch(const fr_hip_batch* req, float* y) {
   // travel in pieces, each on its way while the host copies the next
   // (512 tokens: 1058 us per call with one copy each way, 1020 us in pieces).
   const bool staged = used <= kBatchStaged;
+  sent = true;
   if (staged) {
     memcpy(E.bplan_host + H.x_off, req->x, bytes);
     void* mapped = nullptr;
@@ -7582,10 +7584,11 @@ int fr_hip_run_batch(const fr_hip_batch* req, float* y) {
   if (!g_open) return FR_HIP_STATE;
   if (!req || !y) return FR_HIP_INVALID;
   CK(hipSetDevice(E.device));
-  const int rc = run_batch(req, y);
+  bool sent = false;
+  const int rc = run_batch(req, y, sent);
   // The next call writes the pinned plan and y at once: no copy of a call that
   // fails half-way is left on its way.
-  if (rc) (void)hipStreamSynchronize(E.stream);
+  if (rc && sent) (void)hipStreamSynchronize(E.stream);
   return rc;
 }
 
