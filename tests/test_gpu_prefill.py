@@ -188,56 +188,115 @@ def test_prefill_error_paths(eng):
     eng.release(2)
 
 
-def test_prefill_large_down_scales(eng):
-    """Down super-blocks whose d is 4 or more in magnitude (4, -5, 6, 100, and
-    65504, the largest fp16) in one expert's slice: the down kernel takes those
-    slices on its scaled path; rows against the oracle and against run()."""
-    hidden, blocks = 4096, (0, 1)
+def cut_of(eng, experts, gates, x):
+    """[gslices, gdown] of the plan's BatchHeader: the kernels the chunk takes."""
+    return eng.batch_plan(0, experts, gates, x, fa.MODE_F32)[72:80].view(np.uint32).tolist()
+
+
+def hot_and_cold(experts):
+    """The expert of most tokens and one of the fewest."""
+    count = np.bincount(experts.ravel(), minlength=512)
+    return [int(np.argmax(count)), int(np.flatnonzero(count == count[count > 0].min())[0])]
+
+
+# The chunks below run on prefill_gate_up_few and prefill_down_few, or on
+# prefill_gate_up<4> and prefill_down with tiles of 16 to 64 tokens.
+BOTH = pytest.mark.parametrize("hidden,nblk,tokens,pool,cut", [(4096, 2, 24, 30, [0, 0]), (2560, 20, 320, 300, [4, 1])])
+
+
+@BOTH
+@pytest.mark.parametrize("which", ["d", "dmin"])
+def test_prefill_large_down_scales(eng, hidden, nblk, tokens, pool, cut, which):
+    """Down super-blocks whose d (or dmin) is 4 or more in magnitude (4, -5, 6, 100,
+    and 65504, the largest fp16) in slices of a hot expert and of a cold one, some
+    super-blocks of a slice and slices side by side: with d the down kernels
+    take those slices on their scaled path. The chunk's rows and run()'s against the
+    oracle."""
+    blocks = tuple(range(nblk))
     lay = oracle.layout(hidden, fa.FMT_Q4KT)
     load(eng, hidden, blocks)
     rng = np.random.default_rng(4444)
-    pool = rng.choice(512, 30, replace=False)
-    experts, gates, x = chunk(rng, 24, hidden, pool)
-    e0 = int(experts[2, 3])
-    units = host_units(lay, blocks, 0, experts)
-    view = slice_view(units[1], lay, 0, e0)
-    good = view.copy()
-    for neuron, sb, d in ((5, 3, 0x4400), (17, 9, 0xC500), (0, 0, 0x4600), (31, 15, 0x5640), (12, 6, 0x7BFF)):
-        off = 2 * lay.proj + neuron * lay.down_row + 144 * sb
-        view[off:off + 2] = np.array([d], np.uint16).view(np.uint8)
-    try:
-        assert eng.refresh(1, units[1], 0, e0) == fa.OK
-        y = run_ok(eng, 0, experts, gates, x)
-        rows = []
-        for t0 in range(0, x.shape[0], 8):
-            sl = slice(t0, t0 + 8)
-            rc, ref = oracle.ref_run(units, fa.FMT_Q4KT, False, oracle_request(0, experts[sl], gates[sl], x[sl]))
-            assert rc == 0
-            rows.append(ref[:8])
-        check_close(np.concatenate(rows), y, fa.MODE_F32, "prefill large down scales")
-        check_close(run_bursts(eng, 0, experts, gates, x), y, fa.MODE_F32, "prefill large down scales vs run")
-    finally:
-        view[:] = good
-        assert eng.refresh(1, units[1], 0, e0) == fa.OK
+    experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
+    assert cut_of(eng, experts, gates, x) == cut
+    chosen = hot_and_cold(experts)
+    rows = np.unique(np.concatenate([np.flatnonzero((experts == e).any(axis=1))[:9] for e in chosen] + [np.arange(3)]))
+    units = host_units(lay, blocks, 0, experts[rows])
+    edits = ((5, 3, 0x4400), (17, 9, 0xC500), (0, 0, 0x4600), (31, hidden // 256 - 1, 0x5640), (12, 6, 0x7BFF))
+    for b, e in [(1, chosen[0]), (1, chosen[1]), (nblk - 2, chosen[0])]:
+        view = slice_view(units[b], lay, 0, e)
+        for neuron, sb, v in edits:
+            off = 2 * lay.proj + neuron * lay.down_row + 144 * sb + (2 if which == "dmin" else 0)
+            view[off:off + 2] = np.array([v], np.uint16).view(np.uint8)
+        assert eng.refresh(b, units[b], 0, e) == fa.OK
+    y = run_ok(eng, 0, experts, gates, x)
+    ref = []
+    for i in range(0, len(rows), 8):
+        part = rows[i:i + 8]
+        rc, r = oracle.ref_run(units, fa.FMT_Q4KT, False, oracle_request(0, experts[part], gates[part], x[part]))
+        assert rc == 0
+        ref.append(r[:len(part)])
+    # y is one neuron's h at d = 65504, whose own dot may nearly cancel: a chunk and
+    # run() differ by up to the sum of their distances from the oracle.
+    check_close(np.concatenate(ref), y[rows], fa.MODE_F32, ("prefill large down scales", which))
+    check_close(np.concatenate(ref), run_bursts(eng, 0, experts[rows], gates[rows], x[rows]), fa.MODE_F32, ("run", which))
 
 
-def test_prefill_down_operand_parts_agree(eng):
+@pytest.mark.parametrize("seed,blocks,tokens,pool,cut", [
+    (5, (0, 1), 40, 40, [0, 0]), (6, (0, 1), 40, 40, [0, 0]), (7, (3,), 40, 40, [0, 0]),
+    (5, tuple(range(20)), 320, 300, [4, 1]), (6, tuple(range(20)), 320, 300, [4, 1]),
+])
+def test_prefill_down_operand_parts_agree(eng, seed, blocks, tokens, pool, cut):
     """The down's two f16 parts of d*h sum to it: every token within 2e-6 of the
-    oracle. fp32 sums of 20 terms whose magnitudes add up to a few times the
-    result leave about 1e-6 at most; a hi part that one use rounds differently
-    from the other (2^-11 of one product) shows as 3e-6 and more in some token
-    of each of these chunks."""
+    oracle (of a large chunk, 40 of them). fp32 sums of 20 terms whose magnitudes
+    add up to a few times the result leave about 1e-6 at most; a hi part that one
+    use rounds differently from the other (2^-11 of one product) shows as 3e-6
+    and more in some token of each of the small chunks."""
     hidden = 4096
     lay = oracle.layout(hidden, fa.FMT_Q4KT)
-    for seed, blocks in ((5, (0, 1)), (6, (0, 1)), (7, (3,))):
-        load(eng, hidden, blocks)
-        rng = np.random.default_rng(seed)
-        experts, gates, x = chunk(rng, 40, hidden, rng.choice(512, 40, replace=False))
-        y = run_ok(eng, 0, experts, gates, x)
-        ref = oracle_rows(lay, blocks, 0, experts, gates, x)
-        for t in range(len(x)):
-            rc, err = oracle.compare(ref[t], y[t])
-            assert rc == 0 and err[0] <= 2e-6, (seed, t, err)
+    load(eng, hidden, blocks)
+    rng = np.random.default_rng(seed)
+    experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
+    assert cut_of(eng, experts, gates, x) == cut
+    y = run_ok(eng, 0, experts, gates, x)
+    rows = np.arange(40) * (tokens // 40)
+    ref = oracle_rows(lay, blocks, 0, experts[rows], gates[rows], x[rows])
+    for i, t in enumerate(rows):
+        rc, err = oracle.compare(ref[i], y[t])
+        assert rc == 0 and err[0] <= 2e-6, (seed, t, err)
+
+
+@BOTH
+def test_prefill_bad_scales_and_x(eng, hidden, nblk, tokens, pool, cut):
+    """A non-finite x, and one non-finite d or dmin in a gate, an up or a down row
+    of the last slice of a hot expert's or a cold one's, each end in FR_NUMERIC
+    with y untouched; the restored chunk is bit-identical."""
+    blocks = tuple(range(nblk))
+    lay = oracle.layout(hidden, fa.FMT_Q4KT)
+    load(eng, hidden, blocks)
+    rng = np.random.default_rng(78)
+    experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
+    assert cut_of(eng, experts, gates, x) == cut
+    good = run_ok(eng, 0, experts, gates, x)
+    for v in (np.inf, np.nan):
+        bad = x.copy()
+        bad[tokens - 1, hidden - 1] = v
+        rc, y = eng.run_batch(0, experts, gates, bad)
+        assert rc == fa.NUMERIC and not y.any()
+    chosen = hot_and_cold(experts)
+    units = host_units(lay, blocks[-1:], 0, chosen)
+    b = blocks[-1]
+    for e in chosen:
+        view = slice_view(units[b], lay, 0, e)
+        keep = view.copy()
+        for off in (0, lay.proj + 31 * lay.gu_row + lay.gu_row - 144 + 2, 2 * lay.proj, 2 * lay.proj + 32 * lay.down_row - 144 + 2):
+            view[off:off + 2] = np.array([0x7C00], np.uint16).view(np.uint8)
+            assert eng.refresh(b, units[b], 0, e) == fa.OK
+            print(f"non-finite scale at {off} of expert {e}", flush=True)
+            rc, y = eng.run_batch(0, experts, gates, x)
+            assert rc == fa.NUMERIC and not y.any(), (e, off)
+            view[:] = keep
+            assert eng.refresh(b, units[b], 0, e) == fa.OK
+    assert np.array_equal(run_ok(eng, 0, experts, gates, x).view(np.uint32), good.view(np.uint32))
 
 
 @pytest.mark.parametrize("hidden,nblk,tokens,pool,slices,down", [
@@ -259,8 +318,7 @@ def test_prefill_gate_up_cuts(eng, hidden, nblk, tokens, pool, slices, down):
     load(eng, hidden, blocks)
     rng = np.random.default_rng(hidden + tokens)
     experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
-    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
-    assert plan[72:80].view(np.uint32).tolist() == [slices, down]   # BatchHeader.gslices, gdown
+    assert cut_of(eng, experts, gates, x) == [slices, down]
     y = run_ok(eng, 0, experts, gates, x)
     assert np.array_equal(y, run_ok(eng, 0, experts, gates, x))
     rows = rng.choice(tokens, 7, replace=False)
@@ -268,8 +326,8 @@ def test_prefill_gate_up_cuts(eng, hidden, nblk, tokens, pool, slices, down):
     check_close(ref, y[rows], fa.MODE_F32, ("cut", hidden, nblk))
 
 
-@pytest.mark.parametrize("tokens", [1, 60, 63, 64, 130, 300])
-def test_prefill_run_batch_equals_resident_plan(eng, tokens):
+@pytest.mark.parametrize("tokens,blocks", [(n, (0, 7)) for n in (1, 60, 63, 64, 130, 300)] + [(520, tuple(range(20)))])
+def test_prefill_run_batch_equals_resident_plan(eng, tokens, blocks):
     """fr_hip_run_batch's way up and down (copy kernels up to 1 MB of plan, which
     64 tokens at hidden 4096 pass; 512 KB pieces above) leaves y what a resident
     plan gives, bit for bit; and after a call that fails, fr_hip_batch_output
@@ -278,9 +336,10 @@ def test_prefill_run_batch_equals_resident_plan(eng, tokens):
 
     import torch
     hidden = 4096
-    load(eng, hidden, (0, 7))
+    load(eng, hidden, blocks)
     rng = np.random.default_rng(tokens)
     experts, gates, x = chunk(rng, tokens, hidden)
+    assert cut_of(eng, experts, gates, x) == ([0, 0] if tokens < 100 else [2, 0] if tokens < 500 else [4, 1])
     y = run_ok(eng, 0, experts, gates, x)
     plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
     dev = torch.from_numpy(plan).to("cuda")
@@ -382,30 +441,28 @@ def test_prefill_buffers_count_as_hot_allocations(eng):
         assert eng.sample().hot_allocations == 6
 
 
-@pytest.mark.parametrize("nblk,tokens,pool,slices", [(20, 320, 300, 4), (2, 24, 30, 0)])
+@BOTH
 @pytest.mark.parametrize("what", ["min", "both"])
-def test_prefill_small_down_scales(eng, what, nblk, tokens, pool, slices):
+def test_prefill_small_down_scales(eng, what, hidden, nblk, tokens, pool, cut):
     """The down of an expert whose fp16 scales are the smallest there are (d and
     dmin 2^-24 to 3 * 2^-24, or d zero and y the min terms alone), on the tokens
     for which it is the only expert with a gate. The main sum has operands of 22
     bits and fp32 sums, the min terms are fp32: at most 2e-6 of a row, as with
     larger scales (operands with f16's absolute floor of 2^-25 would be off by
     2^-13 and more of their largest)."""
-    hidden, blocks = 2560, tuple(range(20 - nblk, 20))
+    blocks = tuple(range(20 - nblk, 20))
     lay = oracle.layout(hidden, fa.FMT_Q4KT)
     load(eng, hidden, blocks)
     rng = np.random.default_rng(31 + nblk)
     experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, pool, replace=False))
-    count = np.bincount(experts.ravel(), minlength=512)
-    chosen = [int(np.argmax(count)), int(np.flatnonzero(count == count[count > 0].min())[0])]   # a hot and a cold one
+    chosen = hot_and_cold(experts)
     rows = []
     for e in chosen:
         for t in np.flatnonzero((experts == e).any(axis=1))[:10]:
             if int(t) not in rows:
                 gates[t, :10] = np.where(experts[t] == e, gates[t, :10], 0)
                 rows.append(int(t))
-    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
-    assert plan[72:80].view(np.uint32).tolist() == [slices, 1 if slices else 0]   # BatchHeader.gslices, gdown
+    assert cut_of(eng, experts, gates, x) == cut
     units = host_units(lay, blocks, 0, chosen)
     try:
         for b in blocks:
