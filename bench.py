@@ -521,8 +521,8 @@ def bench_prefill(args):
         "roofline": {"bound": "hbm", "achieved": round(m["achieved"], 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(m["achieved"] / HBM_PEAK_GBS, 4), "traffic": m["traffic"],
                      "traffic_note": "HBM bytes per layer launch: " + m["traffic_note"],
-                     "kernel": ("prefill_split + prefill_gate_up_rows<Q4_K> + prefill_gate_up_rows<Q8_0> + "
-                                "prefill_down_rows<MXFP4> + prefill_down_rows<Q8_0> + prefill_reduce per layer"
+                     "kernel": ("prefill_split + prefill_gate_up_rows + prefill_down_rows (the shared expert's tiles "
+                                "in the same launches) + prefill_reduce per layer"
                                 if native else
                                 "prefill_split + prefill_gate_up + prefill_down + prefill_reduce per layer")},
         "mfma": {"achieved": round(m["tflops"], 2), "peak": MFMA_F16_PEAK_TFLOPS,

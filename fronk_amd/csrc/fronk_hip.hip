@@ -4000,10 +4000,13 @@ __global__ void synth_kernel(uint8_t* __restrict__ dst, SliceShape routed, Slice
 //   prefill_gate_up  (tile, slices): a, u of up to 64 tokens over the 32
 //                    neurons of up to four slices on f16 matrix cores
 //                    (operands exact), then gate*SiLU(a)*u;
-//   prefill_down     (tile, 512 outputs): the expert's down matrix over all
-//                    owned slices applied to the tile's h on f16 matrix
-//                    cores (A = sc*q exact, B = d*h in two exact parts), one
+//   prefill_down     (tile, 256 outputs): the expert's down matrix over all
+//                    owned slices applied to the h of up to 64 tokens on f16
+//                    matrix cores (A = sc*q exact, B = d*h in two parts), one
 //                    fp32 partial per (token, expert);
+//   the same two with smaller workgroups where prefill_cut finds them faster
+//                    (prefill_gate_up_few, prefill_down_few), and on the row
+//                    format (prefill_gate_up_rows, prefill_down_rows);
 //   prefill_reduce   (token, 1024 outputs): the token's 10 expert partials
 //                    (then the shared expert's) summed in its routing order
 //                    in fp64, then narrowed with the reference's rule
@@ -4183,7 +4186,9 @@ __device__ __forceinline__ f16x8 nib_octet(uint32_t w, const NibScale& c, const 
 // across them touches every bank once.
 constexpr int kXhRow = 528;
 
-struct GateUpLds {
+// LDS of the gate/up kernels whose x' passes registers (prefill_gate_up_few, the
+// row format's).
+struct StagedX {
   uint8_t xh[2][2][kTileTokens][kXhRow];     // [buffer][part][token][256 f16]: one super-block of x'
   float xs[2][kTileTokens][8];               // sub-block sums of x'
   float main[kDecodeWaves][16][kTileTokens]; // [wave][row][token] scale-weighted dot part
@@ -4220,7 +4225,8 @@ struct GateUpLds {
 // of f16 products.
 constexpr int kGateUpThreads = 256;
 constexpr int kGateUpHalf = kGateUpTiles * 8 * 1024;   // bytes of x' of half a super-block: [tile][part][v][lane][16 B]
-struct GateUpLds2 {
+// LDS of prefill_gate_up: x' comes straight from memory.
+struct GateUpLds {
   uint8_t x[2][kGateUpHalf];                 // from LDS offset 0: the copies address 64 KB
   uint8_t xs[2][kGateUpTiles * 1024];        // [super-block parity][tile][lane][16 B] the sums' parts
 };
@@ -4245,7 +4251,7 @@ __device__ __forceinline__ void gate_up_wait() {
 
 template <int MT, int NB>
 __device__ __forceinline__ void gate_up_tile(const BatchHeader& H, const BatchScratch& S, const BatchTile& T,
-                                             const BatchSlot* slots, unsigned brank0, GateUpLds2& L, uint32_t& bad) {
+                                             const BatchSlot* slots, unsigned brank0, GateUpLds& L, uint32_t& bad) {
   const unsigned nsb = H.hidden / 256, nblk = H.nblk;
   const int lane = threadIdx.x & 63;
   const unsigned wave = uniform(threadIdx.x >> 6), kg = (unsigned)lane >> 4, col = (unsigned)lane & 15;
@@ -4446,7 +4452,7 @@ __global__ __launch_bounds__(kGateUpThreads, 2) void prefill_gate_up(const uint8
   if (tile >= H.ngtiles) return;
   const BatchTile T = reinterpret_cast<const BatchTile*>(plan + H.gtiles_off)[tile];
   const BatchSlot* slots = reinterpret_cast<const BatchSlot*>(plan + H.slots_off) + T.slot0;
-  __shared__ __align__(16) GateUpLds2 L;
+  __shared__ __align__(16) GateUpLds L;
   uint32_t bad = 0;
   switch ((T.ntok + kTileTokens - 1) / kTileTokens) {
     case 1: gate_up_tile<1, NB>(H, S, T, slots, brank0, L, bad); break;
@@ -4480,7 +4486,7 @@ __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_few(const ui
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned rb = (unsigned)wave & 3, p = (unsigned)wave >> 2, kg = (unsigned)lane >> 4,
                  col = (unsigned)lane & 15;
-  __shared__ __align__(16) GateUpLds L;
+  __shared__ __align__(16) StagedX L;
   // Staging: thread -> token tl, 32-byte piece c of its 1 KB of x'.
   const unsigned tl = (unsigned)tid >> 5, c = (unsigned)tid & 31;
   const bool live = tl < T.ntok;
@@ -4649,7 +4655,7 @@ __device__ __forceinline__ void split_bf16(const float (&v)[8], bf16x8& b1, bf16
 // with the matrix units' 0.2 (0.35) beside them; four workgroups per CU (a
 // fourth is worth 12 % even at the price of a few spilled registers with 64
 // tokens). Measured, 20 slices at hidden 4096, against prefill_down_few:
-// 512 tokens 200 (215) us, 4096 tokens 730 (1100) us.
+// 512 tokens 202 (215) us, 4096 tokens 745 (1100) us.
 constexpr float kDownDirect = 4.f;
 constexpr uint32_t kDownSmall = 0x1c00;      // bits of the f16 2^-8
 constexpr int kDownThreads = 256, kDownWaves = kDownThreads / 64;
@@ -4663,12 +4669,12 @@ struct DownLds {
   uint32_t deferred;                         // slices with a large d or dmin (bit R)
 };
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
 // v as two f16 values hi = f16(v), lo = f16(v - hi) (v - hi is exact in fp32).
 // v is opaque to the compiler: a v that is a product would otherwise be
 // rounded to f16 straight from the exact product (v_fma_mixlo_f16) in one use
 // of hi and by way of fp32 in the other, and where the two roundings differ
 // hi + lo is off by 2^-11 of v (one super-block of y by up to 8e-5, measured).
-typedef float f32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void split_f16(const float (&v)[8], f16x8& hi, f16x8& lo) {
   u32x4 h, l;
 #pragma unroll
@@ -5208,16 +5214,16 @@ __global__ __launch_bounds__(kDownThreads, 3) void prefill_down_few(const uint8_
 // and the shared expert of every format (Q8_0 rows, Q8_0 down [H x 32]),
 // kept in the row layout the row-format decode kernel reads (row: [chunk]
 // [16 B] halves, then the scales; a chunk is 64 columns). Same tiles, x'
-// and h scratch as prefill_gate_up / prefill_down.
+// and h scratch as prefill_gate_up_few / prefill_down_few.
 //
 // Gate/up (tile, slice): wavefront w takes row-block w%4 (the gate rows of
 // neurons 8rb..8rb+7, then their up rows) and chunks 2(w/4), 2(w/4)+1 of
 // every super-block; one v_mfma_f32_16x16x32_f16 per 32-column sub-block,
 // lane 16kg + i holding values 8kg..8kg+7 of row i: B exact in f16 (Q4_K:
-// sc*q, nib_pair_sc; Q8_0: q), A = x' in two f16 parts (tokens as rows, so
+// sc*q, nib_pair_at; Q8_0: q), A = x' in two f16 parts (tokens as rows, so
 // that a lane's results are its own row's). Q4_K: the super-block is scaled
 // by d once and the min terms take one fp32 MFMA per four sub-blocks, as in
-// prefill_gate_up; Q8_0: each sub-block's product is scaled by its row's d.
+// prefill_gate_up_few; Q8_0: each sub-block's product is scaled by its row's d.
 __device__ __forceinline__ uint32_t int8_pair_f16(uint32_t v, uint32_t sel) {
   // Bytes of v (signed int8) as two exact f16: 1024 + 128 + q formed in the
   // bits, less 1152.
@@ -5235,7 +5241,7 @@ __device__ __forceinline__ uint32_t int8_pair_f16(uint32_t v, uint32_t sel) {
 constexpr unsigned kRowPad = 272;
 template <bool Q4>
 struct GateUpRowsLds {
-  GateUpLds x;
+  StagedX x;
   uint8_t wq[Q4 ? 64 * kRowPad : 16];
   uint4 wh[Q4 ? 64 * 2 : 1];
 };
@@ -5254,7 +5260,7 @@ __device__ __forceinline__ void gate_up_rows_tile(const uint8_t* __restrict__ pl
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const unsigned rb = (unsigned)wave & 3, p = (unsigned)wave >> 2, kg = (unsigned)lane >> 4,
                  col = (unsigned)lane & 15, i = col;
-  GateUpLds& L = LL.x;
+  StagedX& L = LL.x;
   uint8_t* WQ = LL.wq;
   uint4* WH = LL.wh;
   // x' staging, as prefill_gate_up_few: thread -> token tl, 32-byte piece c.
@@ -5496,7 +5502,10 @@ __device__ __forceinline__ void gate_up_rows_tile(const uint8_t* __restrict__ pl
 // The native chunk's gate/up, shared expert's tiles (the longer ones) first and
 // the routed tiles in the same launch: the shared expert's alone are too few
 // to fill the chip (37 tokens, 7 slices: a launch of its own takes 19 us beside
-// the routed one's 43 us).
+// the routed one's 43 us). Where they do, one launch loses nothing (20 slices,
+// hidden 4096, the shared expert on every token: 512 tokens 1000 us a call with
+// launches of their own, 963 together; 2048 tokens 3000 both ways), though the
+// down's then run at the MXFP4 tiles' four wavefronts per SIMD instead of two.
 __global__ __launch_bounds__(kBatchThreads, 4) void prefill_gate_up_rows(const uint8_t* __restrict__ plan, BatchScratch S) {
   const BatchHeader& H = *reinterpret_cast<const BatchHeader*>(plan);
   __shared__ __align__(16) GateUpRowsLds<true> L;
@@ -7512,8 +7521,10 @@ static int run_batch(const fr_hip_batch* req, float* y, bool& sent) {
   // Small plans travel by copy kernels, whose start costs less than a DMA
   // engine's (37 tokens, hidden 2560: 150 us per call by DMA, 7 us of them per
   // copy and 45 us between the copies and the kernels). Larger ones
-  // travel in pieces, each on its way while the host copies the next
-  // (512 tokens: 1058 us per call with one copy each way, 1020 us in pieces).
+  // travel in pieces, each on its way while the host copies the next (512 tokens:
+  // 1058 us per call with one copy each way, 1020 us in pieces). On both sides of
+  // the line, hidden 4096 and two slices: 62 tokens 185 us by kernel (194 with one
+  // DMA copy each way), 66 tokens 214 us in pieces (215), 256 tokens 491 (508).
   const bool staged = used <= kBatchStaged;
   sent = true;
   if (staged) {

@@ -108,6 +108,24 @@ def test_prefill_rows_match_oracle(eng, fmt, hidden, tokens, blocks, shared_ever
     check_close(run_bursts(eng, 0, experts, gates, x), y, fa.MODE_F32, ("prefill rows vs run", fmt, hidden))
 
 
+def test_prefill_q4kt_with_shared_expert_on_large_tiles(eng):
+    """Q4_K-T units whose chunk takes prefill_gate_up<4> and prefill_down, with the
+    shared expert on every third token (seven shared tiles, the last partial):
+    sampled rows, with and without it, against the oracle; a repeat bit for bit."""
+    hidden, tokens, blocks = 2304, 320, tuple(range(20))
+    lay = oracle.layout(hidden, fa.FMT_Q4KT)
+    load(eng, hidden, blocks, fa.FMT_Q4KT)
+    rng = np.random.default_rng(hidden + tokens + fa.FMT_Q4KT)
+    experts, gates, x = chunk(rng, tokens, hidden, rng.choice(512, 300, replace=False), 3)
+    plan = eng.batch_plan(0, experts, gates, x, fa.MODE_F32)
+    assert plan[72:80].view(np.uint32).tolist() == [4, 1]   # BatchHeader.gslices, gdown
+    y = run_ok(eng, 0, experts, gates, x)
+    assert np.array_equal(run_ok(eng, 0, experts, gates, x).view(np.uint32), y.view(np.uint32))
+    rows = np.array([0, 1, 3, 47, 48, 162, 318, 319])
+    ref = oracle_rows(lay, fa.FMT_Q4KT, blocks, 0, experts[rows], gates[rows], x[rows])
+    check_close(ref, y[rows], fa.MODE_F32, "prefill q4kt shared")
+
+
 def test_prefill_native_512_tokens_properties(eng):
     """512 tokens, uniform top-10 over 512 experts, the shared expert on every
     token, 20 owned native slices at H=2560 (the reference's width)."""
