@@ -6733,6 +6733,12 @@ struct PrefillCut {
 PrefillCut prefill_cut(const std::vector<uint32_t>& count, uint32_t pairs, uint32_t ntiles, uint32_t nblk) {
   static const float turn[2][kGateUpTiles] = {{4.3f, 6.3f, 9.6f, 11.4f}, {2.55f, 3.75f, 5.7f, 7.1f}};
   const float slots = 2.f * (float)E.cus;
+  uint32_t having[kMaxBatchTokens / kTileTokens + 1] = {}, most = 0;   // experts of nt 16-token tiles
+  for (uint32_t c : count) {
+    const uint32_t nt = (c + kTileTokens - 1) / kTileTokens;
+    ++having[nt];
+    most = nt > most ? nt : most;
+  }
   PrefillCut best = {0, 0, 0, 0};
   float least = 1.4f * launch_turns((float)(ntiles * nblk), slots);
   for (uint32_t k = 0; k < 2; ++k) {
@@ -6743,12 +6749,12 @@ PrefillCut prefill_cut(const std::vector<uint32_t>& count, uint32_t pairs, uint3
       --cap;
       tiles = 0;
       memset(len, 0, sizeof(len));
-      for (uint32_t c : count) {
-        const uint32_t nt = (c + kTileTokens - 1) / kTileTokens, n = (nt + cap - 1) / cap;
-        if (!n) continue;
-        tiles += n;
-        len[nt / n] += n - nt % n;
-        if (nt % n) len[nt / n + 1] += nt % n;
+      for (uint32_t nt = 1; nt <= most; ++nt) {
+        if (!having[nt]) continue;
+        const uint32_t n = (nt + cap - 1) / cap;
+        tiles += n * having[nt];
+        len[nt / n] += (n - nt % n) * having[nt];
+        if (nt % n) len[nt / n + 1] += nt % n * having[nt];
       }
     } while (cap > 1 && tiles * groups < 4 * E.cus);
     float mean = 0.f;
